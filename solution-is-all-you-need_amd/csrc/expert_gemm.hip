@@ -1,6 +1,6 @@
-// expert_gemm.hip -- grouped int4 (Q4_0) expert SwiGLU FFN for gfx950,
-// prefill regime: each expert segment is dense enough (tens to hundreds of
-// tokens) to be a real GEMM, so the work runs on the matrix cores.
+// expert_gemm.hip -- grouped int4 (Q4_0) expert SwiGLU FFN for gfx950 on the
+// matrix cores: every expert segment of a few positions or more runs as a GEMM
+// (gemm_regime).
 //
 // Reference operator: kernels/sparse_moe/sparse_matmul.cu:120-215 and its
 // dense branch (:322-365, cuBLAS GEMMs for gate/up and down, SwiGLU between),
@@ -9,49 +9,61 @@
 // Operands are exact, as in the decode regime, and fp16 for
 // v_mfma_f32_16x16x32_f16, so the products are exact and only the fp32
 // accumulation rounds:
-//   A  gate/up: x rounded bf16 -> fp16 by the router's prep (exact for
-//      2^-17 <= |x| < 65504, the fp16 range a bf16 value fits); down: h as
-//      the fp16 pair hi + lo written by the gate/up epilogue
+//   A  gate/up: x as fp16, each token scaled by the power of two that puts its
+//      largest element in [2^14, 2^15) (the router's prep; undone in the
+//      epilogue), so bf16 values down to 2^-32 of the largest are exact; down:
+//      h as the fp16 pair hi + lo written by the gate/up epilogue
 //      (|h - hi - lo| <= 2^-22 |h|).
 //   B  the integers q = n - 8 as fp16: the nibble becomes the fp16 value
-//      1024 + n (one v_and_or_b32 per pair) and one v_pk_add_f16 gives q.
+//      1024 + n (or 1024 + 16 n) by one v_and_or_b32 per pair, and one packed
+//      fp16 add (or fma) gives q.
 // Per 32-group g, an MFMA gives the exact group sums P = A . q (fp32), and
 // acc += d[n][g] * P scales them in fp32 (four FMAs per MFMA output tile).
 // (Weights rounded to fp16 as q * d, one MFMA and no scaling, cost 9e-3 of
 // max-abs error on outputs of magnitude 40 per rounded stage; the layer
 // tolerance is 1e-2.)
 //
-// Tile pipeline.  Both operands are staged by direct-to-LDS loads into a ring
-// of kG2Stages LDS stages two K quads ahead of the MFMAs: per quad, waves 0-3
-// copy the A rows and the B operands (nibbles and scales) of all eight waves,
-// so waves 4-7 never wait on vmcnt and their global stores stay in flight.
-// The loads are issued from inline assembly (dma_b128_unseen), so the
-// compiler adds no waits of its own; per quad there is one workgroup barrier,
-// preceded by each copying wave's wait for its copies of the quad about to
-// be read (the newer quad's copies stay in flight), which also guarantees
-// every wave has left the stage about to be refilled.  A rows are stored with unit s of row
-// r at s ^ a_swizzle(r & 15), so that no ds_read_b128 of the A operands
-// has a bank conflict (see a_swizzle).  Padded groups of K (a ragged last quad of H or I) are
-// skipped.
+// What bounds it.  The scaling is the kernel's floor beside the weights'
+// bytes: a wave issues one vector or matrix instruction per four cycles, an
+// MFMA keeps its unit busy for sixteen, so MFMA + four FMAs is twenty cycles
+// per 16 x 16 x 32 product.  With operands in registers that pattern reaches
+// 1.2 PFLOP/s (gate/up) and 0.75 PFLOP/s (down, two MFMAs a product) here;
+// plain MFMAs reach 1.5.
 //
-// Tiling.  A workgroup of kG2Waves waves owns BM consecutive positions of
-// one expert segment and a block of weight rows; every wave multiplies all BM
-// positions with NB = 2 weight row tiles of its own, so each B operand feeds
-// up to BM / 16 (times AW) MFMAs, one per 16-position tile that holds a
-// segment position.
-//   gate/up (BM 128, AW 1): wave w takes the gate and the up operand of one
-//            16-row tile of I, so its SwiGLU epilogue has both factors of
-//            every output; the workgroup's 8 tiles are 4 whole 32-groups of
-//            I, written as down-operand chunks (hi + lo) via LDS, stored by
-//            waves 4-7.
-//   down (BM 64, AW 2):  wave w takes two 16-row tiles of H.
+// Two workgroups of four waves per CU.  A workgroup owns BM consecutive
+// positions of one expert segment and 4 x 2 row tiles of weights, so a CU
+// always holds two items that share no barrier: one's prologue (item lookup,
+// first copies), epilogue (SwiGLU, stores) and barrier waits run under the
+// other's MFMAs.  (One eight-wave workgroup per CU spent 28% of gate/up and
+// 36% of down outside the K loop at 4096 tokens: all eight waves were in the
+// prologue or the epilogue at the same time.)
 //
-// Schedule.  Per group the wave needs VT (times AW) A operands from LDS; the
-// reads of group g + 1 are issued while the MFMAs of group g run, and the
-// fp32 scaling of a tile's sums runs while the next tile's MFMAs execute, so
-// no instruction waits on the one just issued.  (Left to itself the compiler
-// issued each A read right before its two MFMAs, with a wait for it: one LDS
-// round trip per two MFMAs.)
+// Operand ring.  Both operands come by direct-to-LDS loads, issued from inline
+// assembly (dma_b128_unseen) so that the compiler adds no waits of its own;
+// each wave copies its own weight tiles and a share of the A rows, waits for
+// its copies of the step about to be read, and one workgroup barrier per step
+// publishes them (and says that every wave has left the slot about to be
+// refilled).  A CU's 160 KB give each workgroup 75 KB of ring (RingCfg): with
+// few positions a step is a whole K quad of both operands and the ring is
+// three to five steps deep, which is what streams weights from HBM; at 80
+// positions and more a step is half a quad of A (three slots) and the weights
+// keep a ring of three quads.  A rows are stored with 16-byte unit s of row r
+// at s ^ a_swizzle(r): no ds_read_b128 of A has a bank conflict.
+//
+// Tiling.  Every wave multiplies all BM positions with two weight row tiles of
+// its own, so each B operand feeds one MFMA (down: two) per 16-position tile
+// that holds a segment position.
+//   gate/up (BM 128): wave w takes the gate and the up operand of one 16-row
+//            tile of I, so its epilogue has both factors of every output; the
+//            workgroup's 4 tiles are half a quad of I, written as down
+//            operand units via LDS.
+//   down (BM 64, A rows of hi and lo): wave w takes two 16-row tiles of H.
+//
+// Schedule.  The A reads of group g + 1 are issued while the MFMAs of group g
+// run, and the fp32 scaling of a tile's sums runs while the next tile's MFMAs
+// execute, so no instruction waits on the one just issued.  (Left to itself
+// the compiler issued each A read right before its two MFMAs, with a wait for
+// it: one LDS round trip per two MFMAs.)
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
@@ -66,11 +78,13 @@ namespace pmoe {
 
 struct GemmK {
   SegSrc seg;
-  const uint16_t* a_src;  // fp16 rows [rows][Kq][16 chunks][AW x 8] in MFMA operand order
-  int64_t a_zero_row;     // an all-zero row of a_src
-  int a_by_token;         // 1: A row = token of the position (x); 0: A row = position (h)
+  int32_t* items;         // [8] counters of the item queue, items_stride words apart, cleared by the router
+  int items_stride;
+  const uint16_t* a_src;  // fp16 rows [rows][Kq][half quad][part][group][AW x 8] in MFMA operand order
+  int64_t a_rows;         // rows of a_src
+  const float* a_unscale; // gate/up: per token, the power of two that undoes its scaling
   int64_t Kq;             // quads of K
-  int64_t Kg;             // real 32-groups of K (padded groups of a_src are ignored)
+  int64_t Kg;             // real 32-groups of K (padded groups of a_src are not multiplied)
   int64_t N;              // rows of the weight matrices (I for gate/up, H for down)
   // weights: [E][N/16][Kq][1 KiB] nibbles, [E][N/16][Kq][64] fp16 scales;
   // w1 = gate (or down), w2 = up (gate/up only); sh_* the shared expert's
@@ -82,11 +96,10 @@ struct GemmK {
   const uint16_t* sh_sc1;
   const uint8_t* sh_nib2;
   const uint16_t* sh_sc2;
-  // gate/up output: h as fp16 hi + lo [rows + 1][KqI][16 chunks][hi 8, lo 8],
+  // gate/up output: h as fp16 hi + lo [rows][KqI][half quad][part][group][hi 8, lo 8],
   // the down GEMM's A operand
   uint16_t* hq16;
   int64_t KqI;
-  int64_t h_zero_row;
   // down output: fp32 [rows][H]
   float* outbuf;
 };
@@ -95,14 +108,20 @@ typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 
 // B operand of one 32-group: the lane's four nibble bytes w (bytes 4p..4p+3 of
 // the group's qs for its row) -> the eight fp16 integers n - 8 in kmap order.
-// mask holds 0x000F000F.
+// mask holds 0x000F000F; the nibbles at bits 4..7 need no shift of their own:
+// in place they make 1024 + 16 n, and (1024 + 16 n) / 16 - 72 is n - 8, exactly.
 __device__ inline u32x4 dequant_int_f16(uint32_t w, uint32_t mask) {
   const h2_t off = {(_Float16)1032.0f, (_Float16)1032.0f};
-  const uint32_t r[4] = {and_or(w, mask, 0x64006400u), and_or(w >> 4, mask, 0x64006400u),
-                         and_or(w >> 8, mask, 0x64006400u), and_or(w >> 12, mask, 0x64006400u)};
+  const h2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+  const h2_t off16 = {(_Float16)-72.0f, (_Float16)-72.0f};
+  const uint32_t w8 = w >> 8, mask16 = mask << 4;
+  auto h2 = [](uint32_t v) { return __builtin_bit_cast(h2_t, v); };
+  auto bits = [](h2_t v) { return __builtin_bit_cast(uint32_t, v); };
   u32x4 out;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) out[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, r[i]) - off);
+  out.x = bits(h2(and_or(w, mask, 0x64006400u)) - off);
+  out.y = bits(__builtin_elementwise_fma(h2(and_or(w, mask16, 0x64006400u)), sixteenth, off16));
+  out.z = bits(h2(and_or(w8, mask, 0x64006400u)) - off);
+  out.w = bits(__builtin_elementwise_fma(h2(and_or(w8, mask16, 0x64006400u)), sixteenth, off16));
   return out;
 }
 
@@ -114,36 +133,65 @@ __device__ inline float swiglu_fast(float g, float u) {
   return g * __builtin_amdgcn_rcpf(1.0f + e) * u;
 }
 
-// Item space: for each active segment u, ceil(len_u / BM) position blocks
-// times n_nb row blocks.  s_mb[u] = first position block of segment u (an
-// exclusive prefix over segments, computed by wave 0).
+// s_waitcnt vmcnt(N) lgkmcnt(0), gfx9 encoding.
+template <int N>
+__device__ inline void wait_vm_lgkm0() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
+// Item space: for each active segment u (active slots come first),
+// ceil(len_u / BM) position blocks times n_nb row blocks.  s_mb[u] = first
+// position block of segment u (an exclusive prefix over segments, by wave 0).
+// All descriptor loads are issued before the scan: a loop over 64 slots at a
+// time paid a memory round trip each, twice (7 us of a launch at 257 slots).
+struct BlockPlan {
+  int n_act, n_mb;
+};
 template <int BM>
-__device__ inline int64_t plan_items(const int4* s_desc, int n_act, int* s_mb) {
+__device__ inline BlockPlan plan_blocks(const SegSrc& seg, int* s_mb, BlockPlan* s_plan) {
+  constexpr int kChunks = (kMaxExperts + 1 + kWave - 1) / kWave;
   if (threadIdx.x < kWave) {
     const int lane = threadIdx.x;
-    int carry = 0;
-    for (int u0 = 0; u0 < n_act; u0 += kWave) {
-      const int u = u0 + lane;
-      const int len = u < n_act ? s_desc[u].z - s_desc[u].y : 0;
-      const int v = (len + BM - 1) / BM;
+    int4 d[kChunks];
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+      const int u = i * kWave + lane;
+      d[i] = seg.desc[u < seg.max_slots ? u : seg.max_slots - 1];
+    }
+    int carry = 0, n_act = 0;
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+      if (i * kWave >= seg.max_slots) break;
+      const int u = i * kWave + lane;
+      const bool act = u < seg.max_slots && d[i].x >= 0;
+      const int v = act ? (d[i].z - d[i].y + BM - 1) / BM : 0;
       int inc = v;
 #pragma unroll
       for (int off = 1; off < kWave; off <<= 1) {
         const int t = __shfl_up(inc, off, kWave);
         if (lane >= off) inc += t;
       }
-      if (u < n_act) s_mb[u] = carry + inc - v;
+      if (act) s_mb[u] = carry + inc - v;
       carry += __shfl(inc, kWave - 1, kWave);
+      n_act += __popcll(__ballot(act));
     }
-    if (lane == 0) s_mb[n_act] = carry;
+    // (loads past the last slot are never used: wait for them here, or the
+    // compiler waits for them, vmcnt(0), in every loop that reuses their
+    // registers)
+    wait_vm_lgkm0<0>();
+    if (lane == 0) {
+      s_mb[n_act] = carry;
+      *s_plan = BlockPlan{n_act, carry};
+    }
   }
-  __syncthreads();
-  return s_mb[n_act];
+  lds_barrier();
+  return BlockPlan{__builtin_amdgcn_readfirstlane(s_plan->n_act), __builtin_amdgcn_readfirstlane(s_plan->n_mb)};
 }
 
 // Segment holding position block mb: the last u with s_mb[u] <= mb (binary
 // search; every lane computes the same answer).
-__device__ inline int segment_of_block(const int* s_mb, int n_act, int64_t mb) {
+__device__ inline int segment_of_block(const int* s_mb, int n_act, int mb) {
   int lo = 0, hi = n_act - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
@@ -162,139 +210,171 @@ __device__ inline int segment_of_block(const int* s_mb, int n_act, int64_t mb) {
 // (its position blocks are neighbours in the range), so both come from HBM
 // about once.  (Blocks dealt round-robin over the XCDs put the 2-3 blocks of
 // a segment on different XCDs, each streaming the segment's weights.)
-struct XcdPlan {
-  int nx, x;
-  int64_t l, nl, b0, n_items;
+//
+// Items are drawn, not dealt: a workgroup starts with item l of its XCD's
+// range and then draws from the range's counter, and from the other ranges'
+// once its own is empty.  Drawing keeps an XCD's workgroups on neighbouring
+// items, so they go on sharing A rows and weights in L2, and evens out items
+// of different cost (a segment's last block may hold one position).  Dealt in
+// rounds against drawn (us, gate/up + down): Qwen3 4096 tokens 316 + 270
+// against 284 + 267, DeepSeek-V3 2048 tokens 2084 + 1643 against 1660 + 1409.
+// With fewer than kDrawRounds rounds of items all are dealt: a drawn item waits
+// for an atomic, which at 64 to 1024 tokens of Qwen3 (three rounds) cost 5 to
+// 8 us a kernel.  The router clears the counters.
+constexpr int kDrawRounds = 4;
+struct ItemQueue {
+  int32_t* next;  // items drawn of each range, `stride` words apart
+  int stride;
+  const int* first;  // LDS: [9] the ranges' first items
+  int nx, x0;        // ranges, this workgroup's own
+  bool drawing;
+  int item, step, end;  // the next item dealt to this workgroup, and the end of those
+  __device__ int workgroups(int x) const { return ((int)gridDim.x - x + nx - 1) / nx; }
+  __device__ int drawn(int x, int t) const {  // the t-th item drawn of range x, or -1 past its end
+    const int i = first[x] + workgroups(x) + t;
+    return i < first[x + 1] ? i : -1;
+  }
+  __device__ int take(int x) const {
+    return __hip_atomic_fetch_add(next + x * stride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // A drawn item, or -1 when every range is empty (one thread).  Other ranges
+  // are looked at before they are drawn from: 512 workgroups drawing from
+  // eight empty ranges cost 40 us at about 10 ns an atomic.
+  __device__ int draw() const {
+    if (!drawing) return -1;
+    const int own = drawn(x0, take(x0));
+    if (own >= 0) return own;
+    int t[8];
+#pragma unroll
+    for (int v = 1; v < 8; ++v)
+      t[v] = v < nx ? __hip_atomic_load(next + (x0 + v) % nx * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    wait_vm_lgkm0<0>();  // as in plan_blocks: some of these are never used
+#pragma unroll
+    for (int v = 1; v < 8; ++v) {
+      const int x = (x0 + v) % nx;
+      if (v >= nx || drawn(x, t[v]) < 0) continue;
+      const int i = drawn(x, take(x));
+      if (i >= 0) return i;
+    }
+    return -1;
+  }
+  // This workgroup's next item (every thread calls it) into *s_item, by
+  // thread 0: the caller reads it after a barrier.
+  __device__ void next_item(int* s_item) {
+    if (threadIdx.x == 0) *s_item = item < end ? item : draw();
+    item = item < end ? item + step : end;
+  }
 };
 
-__device__ inline XcdPlan xcd_plan(int64_t n_mb, int64_t n_nb) {
-  XcdPlan q;
+// s_first: [9] ints of LDS.  Item counts stay far below 2^31: an item writes
+// 32 KB of workspace.
+__device__ inline ItemQueue item_queue(int32_t* next, int stride, int n_mb, int n_nb, int* s_first) {
+  ItemQueue q;
+  q.next = next;
+  q.stride = stride;
+  q.first = s_first;
   q.nx = gridDim.x < 8 ? (int)gridDim.x : 8;
-  q.x = (int)(blockIdx.x % q.nx);
-  q.l = blockIdx.x / q.nx;
-  q.nl = ((int64_t)gridDim.x - q.x + q.nx - 1) / q.nx;
-  q.b0 = n_mb * q.x / q.nx;
-  q.n_items = (n_mb * (q.x + 1) / q.nx - q.b0) * n_nb;
+  q.x0 = (int)(blockIdx.x % q.nx);
+  if ((int)threadIdx.x <= q.nx) s_first[threadIdx.x] = n_mb * (int)threadIdx.x / q.nx * n_nb;
+  lds_barrier();
+  const int f0 = __builtin_amdgcn_readfirstlane(s_first[q.x0]);
+  q.item = f0 + (int)blockIdx.x / q.nx;
+  q.step = q.workgroups(q.x0);
+  const int f1 = __builtin_amdgcn_readfirstlane(s_first[q.x0 + 1]);
+  q.drawing = n_mb * n_nb >= kDrawRounds * (int)gridDim.x;
+  q.end = q.drawing && f0 + q.step < f1 ? f0 + q.step : f1;  // drawing: one dealt item each
   return q;
 }
 
-// Shared prologue of both kernels: descriptors, item plan, and the A row of
-// every position of the tile.
 struct TileCoord {
   int e;
   int64_t m0, end;
   int64_t nb;
 };
 
-// half >= 0: only positions [BM / 2 half, BM / 2 (half + 1)) of the block.
-// The active slots' descriptors in LDS, copied once per launch: read there,
-// an item's set-up issues no global load, after which the compiler would
-// wait for every outstanding store of the wave (the gate/up kernel's storing
-// waves keep theirs in flight into the next item).
-struct SegLds {
-  int e[kMaxExperts + 1], beg[kMaxExperts + 1], end[kMaxExperts + 1];
-};
-
-__device__ inline void seg_to_lds(const SegSrc& seg, int n_act, SegLds* sl) {
-  for (int u = threadIdx.x; u < n_act; u += blockDim.x) {
-    const int4 d = seg.desc[u];
-    sl->e[u] = d.x;
-    sl->beg[u] = d.y;
-    sl->end[u] = d.z;
-  }
+__device__ inline int4 sload_int4(const int4* p) {
+  typedef int v4 __attribute__((ext_vector_type(4)));
+  const v4 v = *(const __attribute__((address_space(4))) v4*)(uintptr_t)uniform_ptr(p);
+  return make_int4(v.x, v.y, v.z, v.w);
 }
 
+// Segment, positions and row block of an item.
 template <int BM>
-__device__ inline TileCoord tile_coord(const GemmK& a, const SegLds* sl, const int* s_mb, int n_act,
-                                       const XcdPlan& xp, int64_t item, int64_t n_nb, int64_t* s_row,
-                                       int half = -1) {
+__device__ inline TileCoord tile_coord(const GemmK& a, const int* s_mb, int n_act, int item, int n_nb) {
   TileCoord c;
-  const int64_t mb = xp.b0 + item / n_nb;
-  c.nb = item % n_nb;
-  const int u = segment_of_block(s_mb, n_act, mb);
-  c.e = __builtin_amdgcn_readfirstlane(sl->e[u]);
-  c.m0 = (int64_t)sl->beg[u] + (mb - s_mb[u]) * BM;
-  c.end = sl->end[u];
-  if (half >= 0) {
-    c.m0 += (int64_t)half * (BM / 2);
-    c.end = c.end < c.m0 + BM / 2 ? c.end : c.m0 + BM / 2;
-  }
-  if (threadIdx.x < BM) {
-    const int64_t pos = c.m0 + threadIdx.x;
-    int64_t row = a.a_zero_row;
-    if (pos < c.end) row = a.a_by_token ? (int64_t)a.seg.seg_tok[pos] : pos;
-    s_row[threadIdx.x] = row;
-  }
-  __syncthreads();
+  const int mb = item / n_nb;
+  c.nb = item - mb * n_nb;
+  const int u = __builtin_amdgcn_readfirstlane(segment_of_block(s_mb, n_act, mb));
+  // a scalar load (the descriptors were written by an earlier launch): a vector
+  // load's wait would also wait for the copies and stores in flight
+  const int4 d = sload_int4(a.seg.desc + u);
+  c.e = d.x;
+  c.m0 = (int64_t)d.y + (int64_t)(mb - __builtin_amdgcn_readfirstlane(s_mb[u])) * BM;
+  c.end = d.z;
   return c;
 }
 
 // ------------------------------------------------------------ the kernels
-constexpr int kGemmBMGateUp = 128;  // segment positions per gate/up tile
-constexpr int kGemmBMDown = 64;     // segment positions per down tile
-constexpr int kG2Waves = 8;
-constexpr int kG2Stages = 3;
-constexpr int kG2AUnits = 2048;  // 16-byte units of A per stage: BM x 16 x AW (128 x 16, 64 x 32)
-constexpr int kG2NB = 2;         // B operands per wave in both kernels
-constexpr int kG2BUnits = kG2Waves * kG2NB * kWave;  // nibbles: one 1 KiB unit row per operand
-constexpr int kG2SUnits = kG2Waves * kG2NB * 8;      // scales: 128 B per operand
-constexpr int kG2StageUnits = kG2AUnits + kG2BUnits + kG2SUnits;
+constexpr int kGateUpBM = 128;  // segment positions per gate/up item
+constexpr int kDownBM = 64;      // and per down item
+constexpr int kG2Waves = 4;
+constexpr int kG2NB = 2;  // weight row tiles per wave in both kernels
+constexpr int kG2BNib = kG2Waves * kG2NB * kWave;          // nibbles: one 1 KiB unit row per operand
+constexpr int kG2BUnits = kG2BNib + kG2Waves * kG2NB * 8;  // and 128 B of scales per operand
+constexpr int kG2BLoads = 2 * kG2NB;                       // weight copies per wave per quad
+constexpr int kG2RingUnits = 4800;  // 75 KB: two workgroups and their tables in a CU's 160 KB
+
+// The ring of a block whose leading VT 16-position tiles are multiplied
+// (16-byte units).
+template <int AW, int VT>
+struct RingCfg {
+  // a step is a quad of both operands (few positions), else half a quad of A
+  static constexpr bool kHalf = AW * VT > 4;
+  static constexpr int kUpr = (kHalf ? 8 : 16) * AW;  // units per A row per step
+  static constexpr int kRpd = kWave / kUpr;           // A rows per copy
+  // A copies per wave per step: only those that reach a multiplied tile
+  static constexpr int kALoads = (16 * VT + kG2Waves * kRpd - 1) / (kG2Waves * kRpd);
+  static constexpr int kAUnits = kALoads * kG2Waves * kWave;
+  // whole quads: slots of the ring; half quads: three A slots and three of B quads
+  static constexpr int kSlot = kAUnits + kG2BUnits;
+  static constexpr int kSlots = kG2RingUnits / kSlot > 5 ? 5 : kG2RingUnits / kSlot;
+  static_assert(kHalf ? 3 * kSlot <= kG2RingUnits : kSlots >= 3, "the ring fits");
+};
 
 // Column swizzle of the A rows in LDS.  gfx950 serves a wave's ds_read_b128
 // in four cycles of 16 lanes, lane l in cycle group (b0 ^ b1 ^ b2, b3) of its
 // quad q = l / 4 (measured: two lanes conflict exactly when they share a
 // group, a 16-byte column of a 256-byte LDS row, and not the row).  Lane
-// (n, p) of an A read takes row n + 16 tt and logical unit AW (4p + gi) (+1);
-// storing logical unit s of row r at s ^ a_swizzle(r & 15) puts the 16 lanes
-// of every group in distinct columns for both kernels (AW 1 and 2), where the
-// plain s ^ (r & 15) left two lanes per column (twice the LDS cycles).
-// a_swizzle swaps bits 1 and 2 of r and folds bit 3 into bit 1.
-__device__ inline uint32_t a_swizzle(uint32_t r) {
-  return (r & 9u) | ((r & 2u) << 1) | (((r & 4u) >> 1) ^ ((r & 8u) >> 2));
+// (n, p) of an A read takes row n + 16 tt and logical unit AW (2p + gi % 2)
+// (+ 8 AW for the quad's second half, + 1 for lo), so in one cycle group p's
+// low bit is n2 ^ n3 (or its complement): unit s of row r at s ^ a_swizzle(r)
+// puts the group's 16 lanes in distinct columns.  UPR 8 (two rows per 256
+// bytes), 16 with AW 1, and 16 or 32 with AW 2 need a map each.
+template <int AW, int UPR>
+__device__ inline uint32_t a_swizzle(uint32_t row) {
+  const uint32_t n = row & 15u;
+  if constexpr (UPR == 8) return ((n >> 2) & 1u) | (n & 2u) | ((n >> 1) & 4u);
+  else if constexpr (AW == 1) return n;
+  else return ((n & 3u) << 2) | (n >> 2);
 }
 
-// s_waitcnt vmcnt(N) lgkmcnt(0), gfx9 encoding.
-template <int N>
-__device__ inline void wait_vm_lgkm0() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
-}
-
-// Active segment count (active slots come first; wave 0 scans, the others
-// wait at the barrier) without copying the descriptors to LDS.
-__device__ inline int count_active(const SegSrc& seg, int* s_nact) {
-  if (threadIdx.x < kWave) {
-    int cnt = 0;
-    for (int u0 = 0; u0 < seg.max_slots; u0 += kWave) {
-      const int u = u0 + (int)threadIdx.x;
-      const bool act = u < seg.max_slots && seg.desc[u < seg.max_slots ? u : 0].x >= 0;
-      cnt += __popcll(__ballot(act));
-    }
-    if (threadIdx.x == 0) *s_nact = cnt;
-  }
-  __syncthreads();
-  return *s_nact;
-}
-
-// The multiply-accumulate of one K quad from LDS stage st into acc (shared
-// by both kernels).  VT: the leading 16-position tiles of the block that are
-// multiplied (the caller passes the number of tiles that hold a segment
-// position); the rest lie past the segment end, so their MFMAs, A reads and
-// scaling are skipped, and their accumulators stay zero and are never
+// The multiply-accumulate of NG consecutive groups (one ring step) into acc,
+// shared by both kernels.  sa: the step's A rows; sb: this wave's nibble units
+// of the quad, ss its scales; g0: the step's first group within the quad (0 or
+// 2).  VT: the leading 16-position tiles of the block that are multiplied (the
+// number that hold a segment position); the rest lie past the segment end, so
+// their MFMAs, A reads and scaling are skipped and their accumulators never
 // stored.  A compile-time count keeps the loop branch-free: a run-time test
-// per tile broke the software pipelining and cost 30%.  RAGGED: groups at or
-// past Kg (uniform) are skipped.  a_unit[gi]: this lane's LDS unit of A group
-// gi (see gemm_tile3).
-template <int BM, int AW, int VT, bool RAGGED>
-__device__ __attribute__((always_inline)) inline void quad_math(const u32x4* st, uint32_t q, uint32_t Kg,
-                                                                const uint32_t (&a_unit)[4], uint32_t mask,
-                                                                f32x4 acc[kG2NB][BM / 16]) {
-  static_assert(VT >= 1 && VT <= BM / 16, "tiles to multiply");
+// per tile broke the software pipelining and cost 30%.  RAGGED: only the first
+// n_valid (uniform) groups are multiplied.
+template <int AW, int VT, int BMT, bool RAGGED>
+__device__ __attribute__((always_inline)) inline void step_math(const u32x4* sa, const u32x4* sb, const uint2* ss,
+                                                                int g0, int n_valid, uint32_t a_lane, uint32_t mask,
+                                                                f32x4 (&acc)[kG2NB][BMT]) {
+  typedef RingCfg<AW, VT> C;
   constexpr int NB = kG2NB;
-  constexpr int UPR = 16 * AW;  // 16-byte units per A row
+  constexpr int NG = C::kHalf ? 2 : 4;
   const int lane = threadIdx.x % kWave;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int n = lane % 16;
   const f32x4 z = {0.f, 0.f, 0.f, 0.f};
   // One group: MFMAs of every tile (hi then lo), the scaling of tile tt - 1
   // after the MFMAs of tile tt.
@@ -316,18 +396,39 @@ __device__ __attribute__((always_inline)) inline void quad_math(const u32x4* st,
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[b][VT - 1] += d[b] * pv[(VT - 1) & 1][b];
   };
+  // logical unit AW (8 (gi / 2) + gi % 2) (+ 1) on top of the lane's own
+  // a_lane = n UPR + (2 AW p ^ a_swizzle(n)): the parts occupy different bits
   auto read_a = [&](int gi, u32x4 (&ah)[VT], u32x4 (&al)[VT]) {
+    const uint32_t u = a_lane ^ (uint32_t)(AW * (8 * (gi >> 1) + (gi & 1)));
 #pragma unroll
     for (int tt = 0; tt < VT; ++tt) {
-      ah[tt] = st[a_unit[gi] + tt * 16 * UPR];
-      if constexpr (AW == 2) al[tt] = st[(a_unit[gi] ^ 1u) + tt * 16 * UPR];
+      ah[tt] = sa[u + tt * 16 * C::kUpr];
+      if constexpr (AW == 2) al[tt] = sa[(u ^ 1u) + tt * 16 * C::kUpr];
       else al[tt] = ah[tt];
     }
   };
-  auto operands = [&](const uint2 (&bs)[NB], const u32x4 (&bw)[NB], int gi, u32x4 (&bq)[NB], float (&d)[NB]) {
+  uint32_t bw[NB][NG];
+  uint32_t bs[NB][NG / 2];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if constexpr (C::kHalf) {
+      const uint2 v = reinterpret_cast<const uint2*>(sb + b * kWave + lane)[g0 >> 1];
+      bw[b][0] = v.x;
+      bw[b][1] = v.y;
+      bs[b][0] = reinterpret_cast<const uint32_t*>(ss + b * 16 + lane % 16)[g0 >> 1];
+    } else {
+      const u32x4 v = sb[b * kWave + lane];
+#pragma unroll
+      for (int gi = 0; gi < NG; ++gi) bw[b][gi] = v[gi];
+      const uint2 s2 = ss[b * 16 + lane % 16];
+      bs[b][0] = s2.x;
+      bs[b][1] = s2.y;
+    }
+  }
+  auto operands = [&](int gi, u32x4 (&bq)[NB], float (&d)[NB]) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const uint32_t s2 = gi < 2 ? bs[b].x : bs[b].y;
+      const uint32_t s2 = bs[b][gi >> 1];
       d[b] = half_bits_to_float((uint16_t)((gi % 2) ? (s2 >> 16) : (s2 & 0xffffu)));
       // the scale as fp32 in a register: the scaling is then v_fmac_f32,
       // not the slower mixed-precision v_fma_mix_f32 the compiler would
@@ -336,329 +437,374 @@ __device__ __attribute__((always_inline)) inline void quad_math(const u32x4* st,
       bq[b] = dequant_int_f16(bw[b][gi], mask);
     }
   };
-  // B operands, then the four groups, the A reads of group gi + 1 issued
-  // before the MFMAs of group gi
-  u32x4 bw[NB];
-  uint2 bs[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    bw[b] = st[kG2AUnits + (w * NB + b) * kWave + lane];
-    bs[b] = reinterpret_cast<const uint2*>(st + kG2AUnits + kG2BUnits + (w * NB + b) * 8)[n];
-  }
   if constexpr (!RAGGED) {
     u32x4 ah[2][VT], al[2][VT];
     read_a(0, ah[0], al[0]);
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
-      if (gi < 3) read_a(gi + 1, ah[(gi + 1) & 1], al[(gi + 1) & 1]);
+    for (int gi = 0; gi < NG; ++gi) {
+      if (gi + 1 < NG) read_a(gi + 1, ah[(gi + 1) & 1], al[(gi + 1) & 1]);
       u32x4 bq[NB];
       float d[NB];
-      operands(bs, bw, gi, bq, d);
+      operands(gi, bq, d);
       group_math(ah[gi & 1], al[gi & 1], bq, d);
     }
   } else {
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
-      if (4 * q + gi >= Kg) break;
+    for (int gi = 0; gi < NG; ++gi) {
+      if (gi >= n_valid) break;
       u32x4 ah[VT], al[VT];
       read_a(gi, ah, al);
       u32x4 bq[NB];
       float d[NB];
-      operands(bs, bw, gi, bq, d);
+      operands(gi, bq, d);
       group_math(ah, al, bq, d);
     }
   }
-}
-
-// The LDS offsets (16-byte units) of lane (n, p)'s A operands of group gi,
-// tile 0: hi at n * UPR + ((p * 4 + gi) * AW ^ a_swizzle(n)), lo at that unit
-// ^ 1 (AW * (p * 4 + gi) is even, so the pair stays adjacent); tile tt adds
-// tt * 16 * UPR.
-template <int AW>
-__device__ inline void a_units(uint32_t (&a_unit)[4]) {
-  const int lane = threadIdx.x % kWave;
-  const uint32_t n = (uint32_t)(lane % 16), p = (uint32_t)(lane / 16);
+  // The sums stay in this step: otherwise the compiler sinks an even step's
+  // scaling below the next barrier, which keeps 128 registers of group sums
+  // alive and leaves its MFMAs nothing to overlap with.
 #pragma unroll
-  for (int gi = 0; gi < 4; ++gi) a_unit[gi] = n * 16 * AW + (((p * 4 + gi) * AW) ^ a_swizzle(n));
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int tt = 0; tt < VT; ++tt) asm volatile("" : "+v"(acc[b][tt]));
 }
 
-// One item's K loop through the LDS ring: both operands staged two quads
-// ahead, one barrier per quad.  CW waves issue the copies: with CW = 8 each
-// wave copies its own B operands and a share of A; with CW = 4 waves 0-3 copy
-// everything (wave w the B operands of waves w and w + 4, rt[o] those of wave
-// w + 4 o) and only they wait on vmcnt, so waves 4-7 may keep global stores
-// in flight through the loop (gfx9 counts loads and stores in one vmcnt, and
-// a wait for a copy would also wait for them).
-template <int BM, int AW, int VT, int CW = kG2Waves>
-__device__ inline void gemm_tile3(const GemmK& a, const int64_t* s_row, u32x4* lds, const i32x4& ar,
-                                  const i32x4 (&nr)[kG2NB], const i32x4 (&sr)[kG2NB],
-                                  const int64_t (&rt)[kG2Waves / CW][kG2NB], f32x4 acc[kG2NB][BM / 16]) {
+// One item's K loop through the LDS ring.  s_row: A row of each position;
+// rt: this wave's row tiles; nr / sr: the resources of their weights.
+template <int AW, int VT, int BMT>
+__device__ __attribute__((always_inline)) inline void gemm_tile(const GemmK& a, const uint32_t* s_row, u32x4* lds,
+                                                                const i32x4& ar, const i32x4 (&nr)[kG2NB],
+                                                                const i32x4 (&sr)[kG2NB], const int64_t (&rt)[kG2NB],
+                                                                f32x4 (&acc)[kG2NB][BMT]) {
+  typedef RingCfg<AW, VT> C;
   constexpr int NB = kG2NB;
-  constexpr int OWN = kG2Waves / CW;          // waves whose B operands a copying wave loads
-  constexpr int UPR = 16 * AW;                // 16-byte units per A row
-  constexpr int RPD = kWave / UPR;            // A rows per direct-to-LDS load
-  constexpr int ND = kG2AUnits / kWave / CW;  // A loads per copying wave per quad
-  static_assert(BM * UPR == kG2AUnits && ND >= 1 && CW * OWN == kG2Waves, "one stage holds the tile");
-  // A load i of the copying waves fills rows [CW RPD i, CW RPD (i + 1)); only
-  // the loads that reach a multiplied tile (rows below 16 VT) are issued: the
-  // rest would copy rows that no MFMA reads (at 64 positions to a
-  // 128-position block, half of the A bytes)
-  constexpr int NDV = (16 * VT + CW * RPD - 1) / (CW * RPD);
-  static_assert(NDV >= 1 && NDV <= ND, "A loads issued");
-  constexpr int kLoads = NDV + 2 * OWN * NB;  // copies per copying wave per quad
   const int lane = threadIdx.x % kWave;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const bool copier = w < CW;
   const uint32_t mask = vgpr_const(0x000F000Fu);
   const uint32_t row_bytes = (uint32_t)(a.Kq * 256 * AW);
-  const uint32_t Kq = (uint32_t)a.Kq;
-  // this wave's A loads j = w + CW * i: lane l fills slot l % UPR of row
-  // j * RPD + l / UPR with logical unit (slot ^ a_swizzle(row & 15))
-  uint32_t voff[ND];
+  const uint32_t Kq = (uint32_t)a.Kq, Kg = (uint32_t)a.Kg;
+  // A copy i of this wave fills rows [j Rpd, (j + 1) Rpd), j = w + 4 i: lane l
+  // the unit l % Upr of row j Rpd + l / Upr, from logical unit (l % Upr) ^ a_swizzle
+  uint32_t voff[C::kALoads];
 #pragma unroll
-  for (int i = 0; i < ND; ++i) {
-    const int j = (copier ? w : 0) + CW * i;
-    const int row = j * RPD + lane / UPR;
-    const int unit = (lane % UPR) ^ (int)a_swizzle((uint32_t)row & 15u);
-    voff[i] = (uint32_t)s_row[row] * row_bytes + (uint32_t)unit * 16u;
+  for (int i = 0; i < C::kALoads; ++i) {
+    const uint32_t row = (uint32_t)((w + kG2Waves * i) * C::kRpd + lane / C::kUpr);
+    const uint32_t unit = (uint32_t)(lane % C::kUpr) ^ a_swizzle<AW, C::kUpr>(row);
+    voff[i] = s_row[row] * row_bytes + unit * 16u;
   }
-  uint32_t a_unit[4];
-  a_units<AW>(a_unit);
+  const uint32_t a_lane = (uint32_t)(lane % 16) * C::kUpr +
+                          ((uint32_t)(lane / 16) * 2u * AW ^ a_swizzle<AW, C::kUpr>((uint32_t)(lane % 16)));
   const uint32_t lds0 = lds_addr(lds);
   auto uni = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
-  auto copy = [&](uint32_t q, uint32_t stage) {
-    if (!copier) return;
-    const uint32_t st = lds0 + stage * (kG2StageUnits * 16);
-    const uint32_t aoff = uni(q * 256u * AW);
+  auto copy_a = [&](uint32_t step, uint32_t unit0) {
+    const uint32_t aoff = uni(step * (uint32_t)(C::kUpr * 16));
 #pragma unroll
-    for (int i = 0; i < NDV; ++i)
-      dma_b128_unseen(ar, uni(st + (uint32_t)(w + CW * i) * kWave * 16), voff[i], aoff);
+    for (int i = 0; i < C::kALoads; ++i)
+      dma_b128_unseen(ar, uni(lds0 + (unit0 + (uint32_t)(w + kG2Waves * i) * kWave) * 16u), voff[i], aoff);
+  };
+  auto copy_b = [&](uint32_t q, uint32_t unit0) {
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-      const int ow = w + CW * o;
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const uint32_t tq = uni((uint32_t)rt[o][b] * Kq + q);
-        dma_b128_unseen(nr[b], uni(st + (uint32_t)(kG2AUnits + (ow * NB + b) * kWave) * 16), (uint32_t)lane * 16u,
-                        tq * kQuadNibBytes);
-        // the 128 scale bytes: eight lanes
-        if (lane < 8)
-          dma_b128_unseen(sr[b], uni(st + (uint32_t)(kG2AUnits + kG2BUnits + (ow * NB + b) * 8) * 16),
-                          (uint32_t)lane * 16u, tq * (kQuadScales * 2));
-      }
+    for (int b = 0; b < NB; ++b) {
+      const uint32_t tq = uni((uint32_t)rt[b] * Kq + q);
+      dma_b128_unseen(nr[b], uni(lds0 + (unit0 + (uint32_t)(w * NB + b) * kWave) * 16u), (uint32_t)lane * 16u,
+                      tq * kQuadNibBytes);
+      // the 128 scale bytes: eight lanes
+      if (lane < 8)
+        dma_b128_unseen(sr[b], uni(lds0 + (unit0 + (uint32_t)kG2BNib + (uint32_t)(w * NB + b) * 8u) * 16u),
+                        (uint32_t)lane * 16u, tq * (kQuadScales * 2));
     }
   };
-  copy(0, 0);
-  if (Kq > 1) copy(1, 1);
-  // quads whose four groups are all real; a ragged last quad (H or I not a
-  // multiple of 128) is done after the loop, so the accumulators keep one
-  // register assignment through it
-  const uint32_t Kq_full = (uint32_t)a.Kg / 4;
-  uint32_t stage = 0;
-  auto top = [&](uint32_t q) {
-    asm volatile("" ::: "memory");
-    if (copier) {
-      if (q + 1 < Kq) wait_vm_lgkm0<kLoads>();  // quad q's copies done, q + 1's may fly
+  auto nib_of = [&](uint32_t unit0) { return lds + unit0 + w * NB * kWave; };
+  auto scale_of = [&](uint32_t unit0) {
+    return reinterpret_cast<const uint2*>(lds + unit0 + kG2BNib + w * NB * 8);
+  };
+  if constexpr (!C::kHalf) {
+    // S slots of one quad each; quads q + 1 .. q + S - 1 in flight behind q
+    constexpr uint32_t S = C::kSlots;
+    constexpr int kLoads = C::kALoads + kG2BLoads;
+    auto copy = [&](uint32_t q, uint32_t slot) {
+      copy_a(q, slot * C::kSlot);
+      copy_b(q, slot * C::kSlot + C::kAUnits);
+    };
+#pragma unroll
+    for (uint32_t i = 0; i + 1 < S; ++i)
+      if (i < Kq) copy(i, i);
+    uint32_t slot = 0;
+    auto top = [&](uint32_t q) {
+      asm volatile("" ::: "memory");
+      const uint32_t left = Kq - 1 - q;  // quads behind q still to come
+      if (left >= S - 2) wait_vm_lgkm0<(int)(S - 2) * kLoads>();
+      else if (S > 4 && left == 2) wait_vm_lgkm0<2 * kLoads>();
+      else if (S > 3 && left == 1) wait_vm_lgkm0<kLoads>();
       else wait_vm_lgkm0<0>();
-    } else {
-      wait_vm_lgkm0<63>();  // LDS only: this wave's stores stay in flight
+      __builtin_amdgcn_s_barrier();  // every copy of quad q is in; quad q - 1's slot is free
+      asm volatile("" ::: "memory");
+      if (q + S - 1 < Kq) copy(q + S - 1, slot == 0 ? S - 1 : slot - 1);
+      const uint32_t u0 = slot * C::kSlot;
+      slot = slot == S - 1 ? 0u : slot + 1u;
+      return u0;
+    };
+    const uint32_t full = Kg / 4;
+    for (uint32_t q = 0; q < full; ++q) {
+      const uint32_t u0 = top(q);
+      step_math<AW, VT, BMT, false>(lds + u0, nib_of(u0 + C::kAUnits), scale_of(u0 + C::kAUnits), 0, 4, a_lane, mask,
+                                    acc);
     }
-    __builtin_amdgcn_s_barrier();  // every copy of quad q is in; stage (q - 1) % 3 is free
-    asm volatile("" ::: "memory");
-    if (q + 2 < Kq) copy(q + 2, stage == 0 ? 2u : stage - 1u);
-    const u32x4* st = lds + stage * kG2StageUnits;
-    stage = stage == kG2Stages - 1 ? 0u : stage + 1u;
-    return st;
-  };
-  for (uint32_t q = 0; q < Kq_full; ++q) quad_math<BM, AW, VT, false>(top(q), q, (uint32_t)a.Kg, a_unit, mask, acc);
-  if (Kq_full < Kq) quad_math<BM, AW, VT, true>(top(Kq_full), Kq_full, (uint32_t)a.Kg, a_unit, mask, acc);
+    if (full < Kq) {
+      const uint32_t u0 = top(full);
+      step_math<AW, VT, BMT, true>(lds + u0, nib_of(u0 + C::kAUnits), scale_of(u0 + C::kAUnits), 0, (int)(Kg % 4),
+                                   a_lane, mask, acc);
+    }
+  } else {
+    // A in three slots of half a quad, two steps ahead; B in three slots of a
+    // quad, two quads ahead, refilled on even steps (before the step's A copies)
+    constexpr uint32_t kB0 = 3 * C::kAUnits;
+    const uint32_t n_steps = (Kg + 1) / 2;
+    copy_b(0, kB0);
+    if (Kq > 1) copy_b(1, kB0 + kG2BUnits);
+    copy_a(0, 0);
+    if (n_steps > 1) copy_a(1, C::kAUnits);
+    uint32_t sa = 0, sb = 0;
+    auto top = [&](uint32_t s, bool odd) {
+      asm volatile("" ::: "memory");
+      // newer than step s's copies: step s + 1's A, and the weights copied before it
+      if (s + 1 >= n_steps) wait_vm_lgkm0<0>();
+      else if (odd && (s >> 1) + 2 < Kq) wait_vm_lgkm0<C::kALoads + kG2BLoads>();
+      else wait_vm_lgkm0<C::kALoads>();
+      __builtin_amdgcn_s_barrier();  // every copy of step s is in; step s - 1's slots are free
+      asm volatile("" ::: "memory");
+      if (!odd && (s >> 1) + 2 < Kq) copy_b((s >> 1) + 2, kB0 + (sb == 0 ? 2u : sb - 1u) * kG2BUnits);
+      if (s + 2 < n_steps) copy_a(s + 2, (sa == 0 ? 2u : sa - 1u) * C::kAUnits);
+    };
+    auto math = [&](auto ragged, bool odd) {
+      const uint32_t ub = kB0 + sb * kG2BUnits;
+      step_math<AW, VT, BMT, decltype(ragged)::value>(lds + sa * C::kAUnits, nib_of(ub), scale_of(ub), odd ? 2 : 0, 1,
+                                                      a_lane, mask, acc);
+      sa = sa == 2 ? 0u : sa + 1u;
+    };
+    const uint32_t full = Kg / 2;  // steps with both groups
+    uint32_t s = 0;
+    for (; s + 1 < full; s += 2) {
+      top(s, false);
+      math(std::false_type(), false);
+      top(s + 1, true);
+      math(std::false_type(), true);
+      sb = sb == 2 ? 0u : sb + 1u;
+    }
+    if (s < full) {
+      top(s, false);
+      math(std::false_type(), false);
+      ++s;
+    }
+    if (s < n_steps) {
+      const bool odd = (s & 1) != 0;
+      top(s, odd);
+      math(std::true_type(), odd);
+    }
+  }
   lds_barrier();  // every wave has left the ring before it is reused
 }
 
-__global__ __launch_bounds__(kG2Waves * kWave) void gemm_gate_up_kernel(GemmK a) {
-  constexpr int BM = kGemmBMGateUp;
+// Multiplies an item with exactly the tiles that hold a position (a block of
+// 65 positions takes 5 tiles, not 8: at about 64 positions an expert,
+// DeepSeek-V3's prefill multiplied half again its positions with rounding to
+// 2, 4 or 8).
+template <int AW, int TT, int VT = 1, typename... Args>
+__device__ __attribute__((always_inline)) inline void gemm_tiles(int vt, Args&&... args) {
+  if constexpr (VT == TT) {
+    gemm_tile<AW, VT, TT>(args...);
+  } else {
+    if (vt == VT) gemm_tile<AW, VT, TT>(args...);
+    else gemm_tiles<AW, TT, VT + 1>(vt, args...);
+  }
+}
+
+__global__ __launch_bounds__(kG2Waves * kWave, 2) void gemm_gate_up_kernel(GemmK a) {
+  constexpr int BM = kGateUpBM;
   constexpr int TT = BM / 16;
-  constexpr int kRows = kG2Waves * 16;  // rows of I per workgroup (kG2Waves / 2 groups)
-  __shared__ u32x4 lds_a[kG2Stages * kG2StageUnits];
+  constexpr int kTiles = kG2Waves;  // row tiles of I per workgroup: half a quad of h,
+  constexpr int kUr = 16;           // 16 units of 16 bytes per position
+  __shared__ u32x4 lds_a[kG2RingUnits];
   __shared__ int s_mb[kMaxExperts + 2];
-  __shared__ int64_t s_row[BM];
-  __shared__ SegLds s_seg;
-  __shared__ int s_nact;
+  __shared__ uint32_t s_row[BM];
+  __shared__ float s_un[BM];
+  __shared__ BlockPlan s_plan;
+  __shared__ int s_first[9], s_item;
   const int lane = threadIdx.x % kWave;
-  const int w = threadIdx.x / kWave;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int n = lane % 16;
   const int p = lane / 16;
-  if (blockIdx.x == 0) {
-    // the all-zero down-operand row read for positions past a segment
-    for (int64_t i = threadIdx.x; i < a.KqI * 256; i += blockDim.x) a.hq16[a.h_zero_row * a.KqI * 256 + i] = 0;
-  }
-  const i32x4 ar = buf_rsrc_words(a.a_src, (uint32_t)((a.a_zero_row + 1) * a.Kq * 256));
-  const int n_act = count_active(a.seg, &s_nact);
-  seg_to_lds(a.seg, n_act, &s_seg);
-  const int64_t n_mb = plan_items<BM>(a.seg.desc, n_act, s_mb);  // its barrier publishes s_seg too
-  const int64_t n_nb = ceil_div(a.N, kRows);
-  const XcdPlan xp = xcd_plan(n_mb, n_nb);
+  const i32x4 ar = buf_rsrc_words(a.a_src, (uint32_t)(a.a_rows * a.Kq * 256));
+  const BlockPlan plan = plan_blocks<BM>(a.seg, s_mb, &s_plan);
+  const int64_t n_tiles = a.N / kRowTile;
+  const int n_nb = (int)ceil_div(n_tiles, kTiles);
+  ItemQueue queue = item_queue(a.items, a.items_stride, plan.n_mb, n_nb, s_first);
   const uint32_t nib_bytes = (uint32_t)(a.N * a.Kq * 64), sc_bytes = (uint32_t)(a.N * a.Kq * 8);
-  // The XCD's items end in a partial round of r = n_items % nl items, which
-  // r of its nl workgroups run while the rest idle.  When 2 r <= nl those r
-  // items run as 2 r halves of BM / 2 positions each (still the XCD's last
-  // items, so their weights are the ones in its L2): the last round then
-  // takes about half an item (at 4096 tokens 8 -> 7.5 item times).
-  const int64_t r_last = xp.n_items % xp.nl;
-  const int64_t n_split = (r_last > 0 && 2 * r_last <= xp.nl) ? r_last : 0;
-  const int64_t n_whole = xp.n_items - n_split;
-  for (int64_t ent = xp.l; ent < xp.n_items + n_split; ent += xp.nl) {
-    const int64_t item = ent < n_whole ? ent : n_whole + (ent - n_whole) / 2;
-    const int part = ent < n_whole ? -1 : (int)((ent - n_whole) % 2);
-    const TileCoord c = tile_coord<BM>(a, &s_seg, s_mb, n_act, xp, item, n_nb, s_row, part);
-    if (c.m0 >= c.end) continue;  // the empty second half of a block of <= BM / 2 positions
-    const int64_t n_tiles = a.N / kRowTile;
-    const int64_t t = c.nb * kG2Waves + w;
-    const int64_t tc = t < n_tiles ? t : n_tiles - 1;  // a tile past I computes, unstored
-    const int64_t t4 = t + 4;                           // wave w + 4's tile, copied by wave w < 4
-    const int64_t tc4 = t4 < n_tiles ? t4 : n_tiles - 1;
+  // positions past the segment repeat its last row (computed, not stored)
+  auto token_of = [&](const TileCoord& t) {
+    const int64_t pos = t.m0 + threadIdx.x;
+    return threadIdx.x < BM ? a.seg.seg_tok[pos < t.end ? pos : t.end - 1] : 0;
+  };
+  queue.next_item(&s_item);
+  lds_barrier();
+  int item = __builtin_amdgcn_readfirstlane(s_item);
+  if (item < 0) return;
+  TileCoord c = tile_coord<BM>(a, s_mb, plan.n_act, item, n_nb);
+  int tok = token_of(c);
+  while (true) {
+    if (threadIdx.x < BM) {
+      s_row[threadIdx.x] = (uint32_t)tok;
+      s_un[threadIdx.x] = a.a_unscale[tok];
+    }
+    lds_barrier();
     const bool routed = c.e < a.seg.E;
-    const i32x4 nr[2] = {buf_rsrc_words(routed ? a.nib1 + (int64_t)c.e * nib_bytes : a.sh_nib1, nib_bytes),
-                         buf_rsrc_words(routed ? a.nib2 + (int64_t)c.e * nib_bytes : a.sh_nib2, nib_bytes)};
-    const i32x4 sr[2] = {
-        buf_rsrc_words(routed ? reinterpret_cast<const uint8_t*>(a.sc1) + (int64_t)c.e * sc_bytes
-                              : reinterpret_cast<const uint8_t*>(a.sh_sc1), sc_bytes),
-        buf_rsrc_words(routed ? reinterpret_cast<const uint8_t*>(a.sc2) + (int64_t)c.e * sc_bytes
-                              : reinterpret_cast<const uint8_t*>(a.sh_sc2), sc_bytes)};
-    const int64_t rt[2][2] = {{tc, tc}, {tc4, tc4}};
+    const i32x4 ng = buf_rsrc_words(routed ? a.nib1 + (int64_t)c.e * nib_bytes : a.sh_nib1, nib_bytes);
+    const i32x4 nu = buf_rsrc_words(routed ? a.nib2 + (int64_t)c.e * nib_bytes : a.sh_nib2, nib_bytes);
+    const i32x4 sg = buf_rsrc_words(routed ? reinterpret_cast<const uint8_t*>(a.sc1) + (int64_t)c.e * sc_bytes
+                                           : reinterpret_cast<const uint8_t*>(a.sh_sc1), sc_bytes);
+    const i32x4 su = buf_rsrc_words(routed ? reinterpret_cast<const uint8_t*>(a.sc2) + (int64_t)c.e * sc_bytes
+                                           : reinterpret_cast<const uint8_t*>(a.sh_sc2), sc_bytes);
+    const i32x4 nr[2] = {ng, nu}, sr[2] = {sg, su};
+    const int64_t t = c.nb * kTiles + w;
+    const int64_t tc = t < n_tiles ? t : n_tiles - 1;  // a tile past I computes, unstored
+    const int64_t rt[2] = {tc, tc};
     f32x4 acc[2][TT];
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) acc[b][tt] = z;
-    const int vt = __builtin_amdgcn_readfirstlane((int)ceil_div(c.end - c.m0, (int64_t)16));
-    // exactly the tiles that hold a position (a block of 65 positions takes 5
-    // tiles, not 8: at about 64 positions an expert, DeepSeek-V3's prefill
-    // multiplied half again its positions with rounding to 2, 4 or 8)
-    switch (vt) {
-      case 1: gemm_tile3<BM, 1, 1, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 2: gemm_tile3<BM, 1, 2, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 3: gemm_tile3<BM, 1, 3, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 4: gemm_tile3<BM, 1, 4, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 5: gemm_tile3<BM, 1, 5, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 6: gemm_tile3<BM, 1, 6, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 7: gemm_tile3<BM, 1, 7, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      default: gemm_tile3<BM, 1, 8, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-    }
+    const int64_t left = c.end - c.m0;
+    const int len = (int)(left < BM ? left : BM);  // positions of the block
+    const int vt = __builtin_amdgcn_readfirstlane((len + 15) / 16);
+    gemm_tiles<1, TT>(vt, a, s_row, lds_a, ar, nr, sr, rt, acc);
+    queue.next_item(&s_item);
 
-    // SwiGLU, then h as the fp16 pair hi + lo into LDS in down-operand chunk
-    // order [group of the workgroup][position][part p'][hi 8, lo 8]: element
-    // cc = half * 16 + n of a group sits at j' = kmap^-1(p', cc), half = w % 2.
+    // SwiGLU, then h as the fp16 pair hi + lo into LDS as the workgroup's half
+    // quad of each position's down operand row: 256 bytes, 16-byte unit
+    // 4 p' + 2 gl + (0 hi, 1 lo) for part p' and group gl.  Element
+    // half * 16 + n of a group sits at j' = kmap^-1(p', .) of part p' = n / 4.
+    // Unit u of position m is stored at u ^ (m / 4 % 4), so the four rows that
+    // a wave's write touches lie in different banks.
     uint16_t* hs = reinterpret_cast<uint16_t*>(lds_a);
-    const int gl = w / 2;  // group of the workgroup this wave's tile belongs to
-    const int half = w % 2;
-    const int pp = n / 4;
+    const int gl = w / 2;  // group of the half quad this wave's tile belongs to
     const int rr = n % 4;
-    const int jj = half == 0 ? ((rr & 1) ? 4 : 0) + (rr >> 1) : ((rr & 1) ? 6 : 2) + (rr >> 1);
-    // tiles past the segment (tt >= vt) hold no position that is stored
+    const int jj = ((rr & 1) ? 4 : 0) + (rr >> 1) + 2 * (w % 2);
+    const int u0 = 4 * (n / 4) + 2 * gl;
+    const int uh = (u0 ^ p) * 8 + jj, ul = ((u0 + 1) ^ p) * 8 + jj;
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
-      if (tt >= vt) break;
+      if (tt >= vt) break;  // tiles past the segment hold no position that is stored
+      const float4 un = reinterpret_cast<const float4*>(s_un)[tt * 4 + p];
+      const float uns[4] = {un.x, un.y, un.z, un.w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int m = tt * 16 + 4 * p + j;
-        const float hv = swiglu_fast(acc[0][tt][j], acc[1][tt][j]);
+        const float hv = swiglu_fast(acc[0][tt][j] * uns[j], acc[1][tt][j] * uns[j]);
         const uint32_t hb = float_to_half_bits(hv);
         const uint32_t lb = float_to_half_bits(hv - half_bits_to_float32(hb));
-        uint16_t* chunk = hs + ((gl * BM + m) * 4 + pp) * 16;
-        chunk[jj] = (uint16_t)hb;
-        chunk[8 + jj] = (uint16_t)lb;
+        uint16_t* row = hs + (tt * 16 + 4 * p + j) * (kUr * 8);
+        row[uh] = (uint16_t)hb;
+        row[ul] = (uint16_t)lb;
       }
     }
     lds_barrier();
-    // the stores from waves 4-7, which issue no copies (see gemm_tile3): they
-    // drain while the next item's copies and MFMAs run
-    constexpr int kGroups = kG2Waves / 2;
-    constexpr int kStoreThreads = kG2Waves / 2 * kWave;
-    for (int cidx = (int)threadIdx.x - kStoreThreads; cidx >= 0 && cidx < kGroups * BM * 4; cidx += kStoreThreads) {
-      const int g2 = cidx / (BM * 4);
-      const int m = (cidx / 4) % BM;
-      const int p2 = cidx % 4;
-      const int64_t g = c.nb * kGroups + g2;  // group of I
-      const int64_t pos = c.m0 + m;
-      if (pos < c.end && 2 * g + 1 < n_tiles) {
-        const u32x4* src = reinterpret_cast<const u32x4*>(hs + ((g2 * BM + m) * 4 + p2) * 16);
-        u32x4* dst = reinterpret_cast<u32x4*>(a.hq16 + ((pos * a.KqI + g / 4) * 16 + p2 * 4 + g % 4) * 16);
-        dst[0] = src[0];
-        dst[1] = src[1];
+    // the next item's tokens are on their way while this one's h is stored
+    item = __builtin_amdgcn_readfirstlane(s_item);
+    const TileCoord cn = item < 0 ? c : tile_coord<BM>(a, s_mb, plan.n_act, item, n_nb);
+    tok = token_of(cn);
+    // 16 lanes store a position's 256 bytes (group 1 of a half quad past I is skipped)
+    const bool two = 2 * (c.nb * 2 + 1) + 1 < n_tiles;
+    for (int cidx = threadIdx.x; cidx < len * kUr; cidx += kG2Waves * kWave) {
+      const int m = cidx / kUr, u = cidx % kUr;
+      if (two || (u & 2) == 0) {
+        const u32x4 v = lds_a[m * kUr + (u ^ ((m >> 2) & 3))];
+        *reinterpret_cast<u32x4*>(a.hq16 + ((c.m0 + m) * a.KqI * 32 + c.nb * kUr + u) * 8) = v;
       }
     }
+    if (item < 0) return;
     lds_barrier();
+    c = cn;
   }
 }
 
-__global__ __launch_bounds__(kG2Waves * kWave) void gemm_down_kernel(GemmK a) {
-  constexpr int BM = kGemmBMDown;
+__global__ __launch_bounds__(kG2Waves * kWave, 2) void gemm_down_kernel(GemmK a) {
+  constexpr int BM = kDownBM;
   constexpr int TT = BM / 16;
   constexpr int NB = kG2NB;
   constexpr int kRows = kG2Waves * 16 * NB;  // rows of H per workgroup
-  __shared__ u32x4 lds_a[kG2Stages * kG2StageUnits];
+  static_assert(BM * kRows / 4 <= kG2RingUnits, "the epilogue's rows fit the ring");
+  __shared__ u32x4 lds_a[kG2RingUnits];
   __shared__ int s_mb[kMaxExperts + 2];
-  __shared__ int64_t s_row[BM];
-  __shared__ SegLds s_seg;
-  __shared__ int s_nact;
+  __shared__ uint32_t s_row[BM];
+  __shared__ BlockPlan s_plan;
+  __shared__ int s_first[9], s_item;
   const int lane = threadIdx.x % kWave;
-  const int w = threadIdx.x / kWave;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int n = lane % 16;
   const int p = lane / 16;
-  const i32x4 ar = buf_rsrc_words(a.a_src, (uint32_t)((a.a_zero_row + 1) * a.Kq * 512));
-  const int n_act = count_active(a.seg, &s_nact);
-  seg_to_lds(a.seg, n_act, &s_seg);
-  const int64_t n_mb = plan_items<BM>(a.seg.desc, n_act, s_mb);  // its barrier publishes s_seg too
-  const int64_t n_nb = ceil_div(a.N, kRows);
+  const BlockPlan plan = plan_blocks<BM>(a.seg, s_mb, &s_plan);
+  const int n_nb = (int)ceil_div(a.N, kRows);
   const int64_t n_tiles = a.N / kRowTile;
-  const XcdPlan xp = xcd_plan(n_mb, n_nb);
+  ItemQueue queue = item_queue(a.items, a.items_stride, plan.n_mb, n_nb, s_first);
   const uint32_t nib_bytes = (uint32_t)(a.N * a.Kq * 64), sc_bytes = (uint32_t)(a.N * a.Kq * 8);
-  for (int64_t item = xp.l; item < xp.n_items; item += xp.nl) {
-    const TileCoord c = tile_coord<BM>(a, &s_seg, s_mb, n_act, xp, item, n_nb, s_row);
+  queue.next_item(&s_item);
+  lds_barrier();
+  int item = __builtin_amdgcn_readfirstlane(s_item);
+  while (item >= 0) {
+    const TileCoord c = tile_coord<BM>(a, s_mb, plan.n_act, item, n_nb);
+    const int64_t left = c.end - c.m0;
+    const int len = (int)(left < BM ? left : BM);  // positions of the block
+    // the block's rows are consecutive; those past the segment repeat its last
+    // (computed, not stored)
+    if (threadIdx.x < BM) s_row[threadIdx.x] = (uint32_t)((int)threadIdx.x < len ? (int)threadIdx.x : len - 1);
+    lds_barrier();
+    const i32x4 ar = buf_rsrc_words(reinterpret_cast<const uint8_t*>(a.a_src) + c.m0 * a.Kq * 512,
+                                    (uint32_t)((int64_t)len * a.Kq * 512));
     const bool routed = c.e < a.seg.E;
     const i32x4 nw = buf_rsrc_words(routed ? a.nib1 + (int64_t)c.e * nib_bytes : a.sh_nib1, nib_bytes);
     const i32x4 sw = buf_rsrc_words(routed ? reinterpret_cast<const uint8_t*>(a.sc1) + (int64_t)c.e * sc_bytes
                                            : reinterpret_cast<const uint8_t*>(a.sh_sc1), sc_bytes);
     const i32x4 nr[NB] = {nw, nw};
     const i32x4 sr[NB] = {sw, sw};
-    // waves 0-3 copy their own operands and wave w + 4's (rt[1])
-    int64_t rt[2][NB];
-#pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const int64_t t = (c.nb * kG2Waves + w + 4 * o) * NB + b;
-        rt[o][b] = t < n_tiles ? t : n_tiles - 1;  // a tile past H computes, unstored
-      }
+    int64_t rt[NB];
     f32x4 acc[NB][TT];
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) acc[b][tt] = z;
-    const int vt = __builtin_amdgcn_readfirstlane((int)ceil_div(c.end - c.m0, (int64_t)16));
-    switch (vt) {
-      case 1: gemm_tile3<BM, 2, 1, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 2: gemm_tile3<BM, 2, 2, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      case 3: gemm_tile3<BM, 2, 3, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-      default: gemm_tile3<BM, 2, 4, 4>(a, s_row, lds_a, ar, nr, sr, rt, acc); break;
-    }
-#pragma unroll
     for (int b = 0; b < NB; ++b) {
       const int64_t t = (c.nb * kG2Waves + w) * NB + b;
-      if (t >= n_tiles) continue;
+      rt[b] = t < n_tiles ? t : n_tiles - 1;  // a tile past H computes, unstored
 #pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        if (tt >= vt) break;
+      for (int tt = 0; tt < TT; ++tt) acc[b][tt] = z;
+    }
+    const int vt = __builtin_amdgcn_readfirstlane((len + 15) / 16);
+    gemm_tiles<2, TT>(vt, a, s_row, lds_a, ar, nr, sr, rt, acc);
+    queue.next_item(&s_item);
+    // The block's outputs through LDS, so that a position's 512 bytes are
+    // stored by 32 consecutive lanes (straight from the accumulators a store
+    // instruction wrote four 64-byte pieces).  64-byte unit u of position m is
+    // stored at u ^ (m / 4 % 4): the four positions of a wave's write lie in
+    // different banks.
+    float* os = reinterpret_cast<float*>(lds_a);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int64_t pos = c.m0 + tt * 16 + 4 * p + j;
-          if (pos < c.end) a.outbuf[pos * a.N + t * 16 + n] = acc[b][tt][j];
-        }
+    for (int tt = 0; tt < TT; ++tt) {
+      if (tt >= vt) break;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        float* row = os + (tt * 16 + 4 * p) * kRows + ((w * NB + b) ^ p) * 16 + n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) row[j * kRows] = acc[b][tt][j];
       }
     }
+    lds_barrier();
+    item = __builtin_amdgcn_readfirstlane(s_item);
+    const int cols = (int)(a.N - c.nb * kRows < kRows ? a.N - c.nb * kRows : kRows);  // a multiple of 32
+    float* out = a.outbuf + c.m0 * a.N + c.nb * kRows;
+    for (int i = threadIdx.x; i < len * (kRows / 4); i += kG2Waves * kWave) {
+      const int m = i / (kRows / 4), u = i % (kRows / 4);  // 16-byte unit u of position m
+      if (4 * u < cols)
+        *reinterpret_cast<u32x4*>(out + (int64_t)m * a.N + 4 * u) = lds_a[m * (kRows / 4) + (u ^ (((m >> 2) & 3) << 2))];
+    }
+    lds_barrier();
   }
 }
 
@@ -668,17 +814,27 @@ bool gemm_regime(int64_t T, int k, int E) {
   return slots >= kGemmMinSlotsPerExpert * seg_max;
 }
 
-static int64_t gemm_max_items(const ExpertArgs& x, int BM, int64_t n_nb) {
-  const int64_t rows = x.T * x.k + (x.has_shared ? x.T : 0);
-  return (ceil_div(rows, BM) + max_active_experts(x)) * n_nb;
+// One launch: position blocks of BM times row blocks of `rows`, on the
+// workgroups resident at once.
+template <typename Kernel>
+static hipError_t launch_tiles(Kernel kernel, const ExpertArgs& x, const GemmK& g, int BM, int rows,
+                               hipStream_t stream) {
+  const int64_t positions = x.T * x.k + (x.has_shared ? x.T : 0);
+  const int64_t max_items = (ceil_div(positions, BM) + max_active_experts(x)) * ceil_div(g.N, rows);
+  hipLaunchKernelGGL(kernel, dim3(resident_grid(kernel, kG2Waves * kWave, max_items)), dim3(kG2Waves * kWave), 0,
+                     stream, g);
+  return hipGetLastError();
 }
 
 hipError_t launch_gemm_gate_up(const ExpertArgs& x, const Workspace& ws, hipStream_t stream) {
   GemmK g = {};
   g.seg = segments_of(x, ws);
+  const GemmItems items = gemm_items(ws, x.T, x.H);
+  g.items = items.counters;
+  g.items_stride = items.stride;
   g.a_src = ws.xq;
-  g.a_zero_row = x.T;
-  g.a_by_token = 1;
+  g.a_rows = x.T;
+  g.a_unscale = ws.xs;
   g.Kq = ceil_div(x.H, kQuad);
   g.Kg = x.H / kGroup;
   g.N = x.I;
@@ -692,19 +848,17 @@ hipError_t launch_gemm_gate_up(const ExpertArgs& x, const Workspace& ws, hipStre
   g.sh_sc2 = x.sh_up_scale;
   g.hq16 = ws.hq;
   g.KqI = ceil_div(x.I, kQuad);
-  g.h_zero_row = x.T * x.k + (x.has_shared ? x.T : 0);
-  const int64_t max_items = gemm_max_items(x, kGemmBMGateUp, ceil_div(x.I, kG2Waves * 16));
-  hipLaunchKernelGGL(gemm_gate_up_kernel, dim3(resident_grid(gemm_gate_up_kernel, kG2Waves * kWave, max_items)),
-                     dim3(kG2Waves * kWave), 0, stream, g);
-  return hipGetLastError();
+  return launch_tiles(gemm_gate_up_kernel, x, g, kGateUpBM, kG2Waves * 16, stream);
 }
 
 hipError_t launch_gemm_down(const ExpertArgs& x, const Workspace& ws, hipStream_t stream) {
   GemmK g = {};
   g.seg = segments_of(x, ws);
+  const GemmItems items = gemm_items(ws, x.T, x.H);
+  g.items = items.counters + 8 * items.stride;
+  g.items_stride = items.stride;
   g.a_src = ws.hq;
-  g.a_zero_row = x.T * x.k + (x.has_shared ? x.T : 0);
-  g.a_by_token = 0;
+  g.a_rows = x.T * x.k + (x.has_shared ? x.T : 0);
   g.Kq = ceil_div(x.I, kQuad);
   g.Kg = x.I / kGroup;
   g.N = x.H;
@@ -713,10 +867,7 @@ hipError_t launch_gemm_down(const ExpertArgs& x, const Workspace& ws, hipStream_
   g.sh_nib1 = x.sh_down_nib;
   g.sh_sc1 = x.sh_down_scale;
   g.outbuf = ws.outbuf;
-  const int64_t max_items = gemm_max_items(x, kGemmBMDown, ceil_div(x.H, kG2Waves * 16 * kG2NB));
-  hipLaunchKernelGGL(gemm_down_kernel, dim3(resident_grid(gemm_down_kernel, kG2Waves * kWave, max_items)),
-                     dim3(kG2Waves * kWave), 0, stream, g);
-  return hipGetLastError();
+  return launch_tiles(gemm_down_kernel, x, g, kDownBM, kG2Waves * 16 * kG2NB, stream);
 }
 
 }  // namespace pmoe

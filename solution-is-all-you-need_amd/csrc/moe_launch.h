@@ -171,6 +171,19 @@ struct Workspace {
   uint8_t* cand = nullptr;          // [E * T] candidate flags, expert-major (two-pass router)
 };
 
+// The item counters of the two GEMM kernels, 8 each, in row T of xq (which the
+// GEMM regime does not read), cleared by the router: a 128-byte line each
+// where the row is long enough.
+struct GemmItems {
+  int32_t* counters;  // [16], stride words apart: gate/up, down
+  int stride;
+};
+inline GemmItems gemm_items(const Workspace& ws, int64_t T, int64_t H) {
+  const int64_t Kpad = (H + 127) / 128 * 128;  // at least 256 bytes a row
+  const int64_t words = Kpad / 32;
+  return {reinterpret_cast<int32_t*>(ws.xq + T * Kpad), (int)(words < kCtlStride ? words : kCtlStride)};
+}
+
 // Batches of at least this many slots use the many-workgroup permute.
 constexpr int64_t kPermMultiSlots = 8192;
 inline int64_t perm_blocks(int64_t n) {
@@ -215,7 +228,7 @@ struct RouteArgs {
   int32_t* topk_idx;
   float* topk_w;
   bool prep_x;       // write ws.xq / ws.xs
-  bool prep_fp16;    // ws.xq as fp16 (GEMM regime) instead of bf16 (GEMV regime)
+  bool prep_fp16;    // ws.xq as scaled fp16 and ws.xs its inverse scale per token (GEMM regime) instead of bf16 and group sums
   bool do_permute;   // write offsets / sorted_slots / slot_pos / active
   int has_shared;    // append the shared-expert segment to offsets / active
   bool want_tiles;   // write ws.tiles / ws.n_tiles (the token-tile gate/up kernel reads them)

@@ -54,7 +54,7 @@ struct RouteK {
   float* xs;
   int64_t Kq;  // quads of H (padded)
   int prep_x;
-  int prep_fp16;  // xq holds fp16 (rounded from bf16) instead of bf16
+  int prep_fp16;  // xq holds the GEMM regime's scaled fp16 copy, xs its inverse scales
   // permute
   int do_permute;
   int has_shared;
@@ -69,6 +69,8 @@ struct RouteK {
   int32_t* tiles;    // token tiles (see kTileWords), or null
   int32_t* n_tiles;
   int32_t* counter;  // select workgroups finished (fused permute); zeroed by the logits launch
+  int32_t* items;  // the GEMM regime's 16 item counters, items_stride words apart, which the logits launch clears; or null
+  int items_stride;
   int fuse_permute;
   // many-slot permute: the select launch counts each slot into
   // perm_cnt[e * perm_nb + slot / perm_chunk] (zeroed by the first route
@@ -418,20 +420,84 @@ __device__ void prep_x_tile(const RouteK& a, int64_t t0, int TT, int part, int n
                    (bf16_bits_to_float(lo[u].y & 0xffffu) + bf16_bits_to_float(lo[u].y >> 16))) +
                   ((bf16_bits_to_float(hi[u].x & 0xffffu) + bf16_bits_to_float(hi[u].x >> 16)) +
                    (bf16_bits_to_float(hi[u].y & 0xffffu) + bf16_bits_to_float(hi[u].y >> 16)));
-      if (a.prep_fp16) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t b2 = v[i];
-          v[i] = float_to_half_bits(bf16_bits_to_float(b2 & 0xffffu)) |
-                 (float_to_half_bits(bf16_bits_to_float(b2 >> 16)) << 16);
-        }
-      }
       sum += __shfl_xor(sum, 4, kWave);
       sum += __shfl_xor(sum, 8, kWave);
       if (valid) {
         *reinterpret_cast<u32x4*>(a.xq + (t * per_tok + cc) * 8) = v;
         if (p == 0) a.xs[t * a.Kq * 4 + g] = sum;
       }
+    }
+  }
+}
+
+// The GEMM regime's copy of one token: fp16 of x times the power of
+// two that puts the token's largest element in [2^14, 2^15), so every bf16
+// value down to 2^-32 of it is exact; the inverse goes to xs[t].  (Unscaled,
+// fp16 overflows from 65520 on and loses bits below 2^-17.)  A token with an
+// infinity or NaN is not scaled.  Layout [t][q][gi / 2][p][gi % 2][8]: the two
+// groups of half a quad are 128 consecutive bytes.
+// NT threads (tid of them; whole waves) share the token; with more than one
+// wave the call has a workgroup barrier and s_mx holds one word per wave.
+template <int NT>
+__device__ inline void prep_x_f16_token(const RouteK& a, int64_t t, int tid, uint32_t* s_mx) {
+  const uint16_t* xr = static_cast<const uint16_t*>(a.x) + t * a.H;
+  constexpr int kBatch = 8;  // loads in flight per thread
+  uint32_t mx = 0;
+  for (int64_t h0 = 0; h0 < a.H; h0 += 4 * NT * kBatch) {
+    uint2 v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int64_t h = h0 + 4 * (u * NT + tid);
+      v[u] = *reinterpret_cast<const uint2*>(xr + (h < a.H ? h : 0));
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const uint32_t m0 = v[u].x & 0x7FFF7FFFu, m1 = v[u].y & 0x7FFF7FFFu;
+      mx = max(max(mx, max(m0 & 0xffffu, m0 >> 16)), max(m1 & 0xffffu, m1 >> 16));
+    }
+  }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, s, kWave));
+  if constexpr (NT > kWave) {
+    if (tid % kWave == 0) s_mx[tid / kWave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT / kWave; ++i) mx = max(mx, s_mx[i]);
+    __syncthreads();  // s_mx may be reused for another token
+  }
+  const int ex = (int)(mx >> 7);  // biased exponent of the largest magnitude
+  const int sc = ex == 255 ? 0 : min(141 - ex, 126);
+  const float up = __builtin_bit_cast(float, (uint32_t)(127 + sc) << 23);
+  if (tid == 0) a.xs[t] = __builtin_bit_cast(float, (uint32_t)(127 - sc) << 23);
+  const int Kg = (int)(a.H / kGroup);
+  const int n = (int)a.Kq * 16;
+  constexpr int kChunks = 4;  // chunks in flight per thread
+  for (int c0 = 0; c0 < n; c0 += kChunks * NT) {
+    uint2 lo[kChunks], hi[kChunks];
+#pragma unroll
+    for (int u = 0; u < kChunks; ++u) {
+      const int c = c0 + u * NT + tid;
+      const int g = 4 * (c >> 4) + 2 * ((c >> 3) & 1) + (c & 1);
+      lo[u] = hi[u] = make_uint2(0u, 0u);
+      if (g < Kg) {
+        const uint16_t* src = xr + (int64_t)g * kGroup + 4 * ((c >> 1) & 3);
+        lo[u] = *reinterpret_cast<const uint2*>(src);
+        hi[u] = *reinterpret_cast<const uint2*>(src + 16);
+      }
+    }
+    auto pair = [&](uint32_t b0, uint32_t b1) {  // two bf16 patterns in the high halves
+      return float_to_half_bits(__builtin_bit_cast(float, b0) * up) |
+             (float_to_half_bits(__builtin_bit_cast(float, b1) * up) << 16);
+    };
+#pragma unroll
+    for (int u = 0; u < kChunks; ++u) {
+      const int c = c0 + u * NT + tid;
+      u32x4 v;
+      v.x = pair(lo[u].x << 16, lo[u].y << 16);
+      v.y = pair(hi[u].x << 16, hi[u].y << 16);
+      v.z = pair(lo[u].x & 0xffff0000u, lo[u].y & 0xffff0000u);
+      v.w = pair(hi[u].x & 0xffff0000u, hi[u].y & 0xffff0000u);
+      if (c < n) *reinterpret_cast<u32x4*>(a.xq + (t * n + c) * 8) = v;
     }
   }
 }
@@ -486,6 +552,7 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
   const int e0 = blockIdx.x * (4 * EW) + w * EW;
   const XT* x = static_cast<const XT*>(a.x);
   if (a.counter && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.counter = 0;
+  if (a.items && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 16) a.items[threadIdx.x * a.items_stride] = 0;
   // The bias of the expert this lane may write, fetched ahead of the GEMV.
   float bias_e = 0.0f;
   if (a.bias) {
@@ -532,8 +599,15 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
       }
     }
     // the MFMA-ordered copy of x, its loads in flight with the first batch's
-    if (c0 == 0 && a.prep_x)
-      prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
+    if (c0 == 0 && a.prep_x) {
+      if (!a.prep_fp16) {
+        prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
+      } else {
+        __shared__ uint32_t s_mx[4];
+        for (int ti = (int)blockIdx.x; ti < TT && t0 + ti < a.T; ti += (int)gridDim.x)
+          prep_x_f16_token<256>(a, t0 + ti, (int)threadIdx.x, s_mx);
+      }
+    }
     if (c0 + CB > nfull) {
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) {
@@ -578,7 +652,7 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
     }
   }
 
-  if (a.prep_x && blockIdx.x == 1 % gridDim.x && blockIdx.y == 0) {
+  if (a.prep_x && !a.prep_fp16 && blockIdx.x == 1 % gridDim.x && blockIdx.y == 0) {
     // all-zero activation row T, read by expert lanes past a segment
     for (int64_t i = threadIdx.x; i < a.Kq * 128; i += blockDim.x) a.xq[a.T * a.Kq * 128 + i] = 0;
     for (int64_t i = threadIdx.x; i < a.Kq * 4; i += blockDim.x) a.xs[a.T * a.Kq * 4 + i] = 0.0f;
@@ -716,8 +790,13 @@ __global__ __launch_bounds__(256) void route_logits_big_kernel(RouteK a) {
   const int64_t t0 = (int64_t)blockIdx.y * TT;
   const int e0 = blockIdx.x * (4 * EW) + w * EW;
   const XT* x = static_cast<const XT*>(a.x);
-  if (a.prep_x) prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
+  if (a.prep_x && !a.prep_fp16)
+    prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
+  if (a.prep_x && a.prep_fp16)
+    for (int ti = (int)blockIdx.x * 4 + w; ti < TT && t0 + ti < a.T; ti += (int)gridDim.x * 4)
+      prep_x_f16_token<kWave>(a, t0 + ti, lane, nullptr);
   if (a.counter && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.counter = 0;
+  if (a.items && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 16) a.items[threadIdx.x * a.items_stride] = 0;
   float bias_e = 0.0f;
   if (a.bias) {
     const int e = e0 + tree_pair_of_lane<P>(lane) % EW;
@@ -841,6 +920,7 @@ __global__ __launch_bounds__(256) void route_approx_kernel(RouteK a, float* appr
   const int e0 = (int)eb * kApproxExp;
   const uint16_t* x = static_cast<const uint16_t*>(a.x);
   if (a.counter && blockIdx.x == 0 && threadIdx.x == 0) *a.counter = 0;
+  if (a.items && blockIdx.x == 0 && threadIdx.x < 16) a.items[threadIdx.x * a.items_stride] = 0;
   if (a.perm_cnt)
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (int64_t)a.E * a.perm_nb;
          i += (int64_t)gridDim.x * blockDim.x)
@@ -986,7 +1066,8 @@ __global__ __launch_bounds__(512) void route_candidates_kernel(RouteK a, const f
     // of H 2048 and 17.5 us at 2048 of H 7168)
     if (a.prep_x)
       for (int64_t t0 = (int64_t)blockIdx.x * 4; t0 < a.T; t0 += (int64_t)gridDim.x * 4)
-        prep_x_tile(a, t0, 4, 0, 1, (int)threadIdx.x - 4 * kWave, 4 * kWave);
+        if (!a.prep_fp16) prep_x_tile(a, t0, 4, 0, 1, (int)threadIdx.x - 4 * kWave, 4 * kWave);
+        else if (t0 + w - 4 < a.T) prep_x_f16_token<kWave>(a, t0 + w - 4, lane, nullptr);
     return;
   }
   for (int64_t t = (int64_t)blockIdx.x * 4 + w; t < a.T; t += (int64_t)gridDim.x * 4) {
@@ -1633,6 +1714,9 @@ hipError_t launch_route(const RouteArgs& r, const Workspace& ws, hipStream_t str
   const unsigned sel_blocks = (unsigned)ceil_div(r.T, kSelectWaves);
   k.fuse_permute = (r.do_permute && sel_blocks > 1 && sel_blocks <= kFusedSelectBlocks) ? 1 : 0;
   k.counter = k.fuse_permute ? ws.counter : nullptr;
+  const GemmItems items = gemm_items(ws, r.T, r.H);
+  k.items = r.prep_x && r.prep_fp16 ? items.counters : nullptr;
+  k.items_stride = items.stride;
   const bool two_pass = two_pass_route(r.T, r.E, r.x_dtype) && ws.approx && ws.cand && !k.fuse_permute;
   // With two passes and a fused scan the select launch does the permute's
   // counting (the approximate-logit launch zeroes the counts first).

@@ -1,0 +1,77 @@
+"""The expert GEMMs at the edges of their tiles: 16-position tiles and blocks
+(64 and 128 positions), row tiles past I and H, ragged K, drawn items, and
+activations outside fp16's own range.  Reference: the fp64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+import phantom_moe
+from oracle import oracle
+from phantom_moe import synth
+from tests.helpers import to_bf16_tensor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+def run(dev, cfg, xb, L):
+    ex = phantom_moe.MoEWeights.from_q4_0(
+        *(torch.from_numpy(a).to(dev) for a in (L.gate, L.up, L.down)), cfg.H, cfg.I, cfg.E,
+        shared=None if L.shared is None else tuple(torch.from_numpy(a).to(dev) for a in L.shared))
+    y, _, idx = phantom_moe.moe_forward(to_bf16_tensor(xb, dev), torch.from_numpy(L.router_w).to(dev), ex, cfg.k,
+                                        cfg.score, return_routing=True)
+    ry, ridx, _ = oracle.moe_forward(xb, L.router_w, L.gate, L.up, L.down, cfg.k, cfg.score_mode, None,
+                                     shared=L.shared)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ridx)
+    y = y.cpu().numpy().astype(np.float64)
+    assert np.isfinite(y).all()
+    # Exact products summed in fp32: every token's error stays within the
+    # (H + I) / 32 group sums' and their 32 products' roundings of 2^-24 each,
+    # taken as independent with room for the cancellation of the sums
+    err = np.linalg.norm(y - ry, axis=1) / np.linalg.norm(ry, axis=1)
+    assert err.max() <= 8 * np.sqrt((cfg.H + cfg.I) / 32 + 32) * 2.0 ** -24, (cfg.name, err.max())
+
+
+# (T, H, I, E, k, shared): T * k >= 64 slots per expert, so the GEMMs run
+CASES = [
+    (64, 128, 32, 1, 1, False),     # one block of four tiles; one row tile pair, the rest past I
+    (65, 160, 96, 1, 1, False),     # H: one whole quad and one group; I: half a quad and one group
+    (81, 192, 160, 1, 1, False),    # six tiles; two groups past a whole quad
+    (112, 224, 128, 1, 1, True),    # seven tiles; three groups past a whole quad
+    (128, 96, 224, 1, 1, False),    # a whole gate/up block; K under a quad
+    (129, 256, 64, 1, 1, False),    # a last block of one position
+    (209, 384, 192, 2, 1, False),   # segments of any length
+    (160, 640, 320, 2, 2, True),    # both experts and the shared one see every token
+    (1100, 512, 1024, 16, 1, False),  # a launch with drawn items
+]
+
+
+@pytest.mark.parametrize("shape", CASES, ids=lambda s: "-".join(str(int(v)) for v in s))
+def test_gemm_edges(dev, shape):
+    T, H, I, E, k, shared = shape
+    cfg = synth.MoEConfig("gemm", H, I, E, k, T, shared=shared)
+    run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg))
+
+
+@pytest.mark.parametrize("T", [64, 130])  # the one-pass and (E 16) the two-pass router's copy of x
+def test_gemm_activation_range(dev, T):
+    """Tokens with elements past fp16's range (65504) beside ones down to
+    2^-34.  |h| must stay under 65504: with weights of at most 8 * 2^-17 and
+    elements spread over 12 octaves below a largest one of at most 2^17.5,
+    |g| and |u| stay under about 4 * 16 / 6 * 2^17.5 * 2^-14 = 2^7, and h
+    under 2^14."""
+    E = 16 if T >= 128 else 1
+    k = 8 if T >= 128 else 1
+    cfg = synth.MoEConfig("range", 256, 64, E, k, T)
+    L = synth.host_layer(cfg)
+    for a in (L.gate, L.up):
+        a[..., 0:2] = np.full(a.shape[:-1] + (1,), 2.0 ** -17, dtype=np.float16).view(np.uint8)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, cfg.H)) * np.exp2(rng.uniform(-12, 0, (T, cfg.H)))
+    x *= np.exp2(rng.uniform(11, 17.5, (T, 1))) / np.abs(x).max(axis=1, keepdims=True)
+    x[:, ::16] *= 2.0 ** -40
+    run(dev, cfg, synth.f32_to_bf16_bits(x.astype(np.float32)), L)
