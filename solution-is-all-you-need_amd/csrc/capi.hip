@@ -381,7 +381,7 @@ int check_forward(ForwardCall& c) {
     return fail(PHANTOM_MOE_EINVAL, "x must be 8-byte and router_w 16-byte aligned");
   // the decode-regime down kernel reads one expert segment's operand (at
   // most T positions of I as fp16 hi and lo) through a 32-bit buffer resource
-  if (!pmoe::gemm_regime(c.T, c.top_k, c.E) && c.T * ((c.I + 127) / 128) * 512 >= ((int64_t)1 << 31))
+  if (!pmoe::dense_segments(c.T, c.top_k, c.E) && c.T * ((c.I + 127) / 128) * 512 >= ((int64_t)1 << 31))
     return fail(PHANTOM_MOE_EUNSUPPORTED, "T*I too large for the decode regime (one segment's down operand above 2 GiB)");
   return 0;
 }
@@ -453,7 +453,7 @@ int run_forward(const ForwardCall& c, void* workspace, hipStream_t stream) {
     }
   }
 
-  const bool gemm = pmoe::gemm_regime(T, top_k, E);
+  const bool gemm = pmoe::gemm_regime(T, H, I, top_k, E, has_shared);
   r.prep_x = true;
   r.prep_fp16 = gemm;
   r.do_permute = true;
@@ -493,7 +493,7 @@ const char* phantom_moe_expert_kernels(int64_t T, int64_t H, int64_t I, int E, i
     gu = dn = fp.spec == pmoe::kFusedSpecX8 ? "moe_decode_x8_kernel" : "moe_decode_fused_kernel";
   } else if (pmoe::stream_plan(T, H, I, E, top_k, has_shared ? 1 : 0).ok) {
     gu = dn = "moe_decode_stream_kernel";
-  } else if (pmoe::gemm_regime(T, top_k, E)) {
+  } else if (pmoe::gemm_regime(T, H, I, top_k, E, has_shared ? 1 : 0)) {
     gu = "gemm_gate_up_kernel";
     dn = "gemm_down_kernel";
   } else {

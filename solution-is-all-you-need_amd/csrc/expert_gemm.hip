@@ -808,10 +808,31 @@ __global__ __launch_bounds__(kG2Waves * kWave, 2) void gemm_down_kernel(GemmK a)
   }
 }
 
-bool gemm_regime(int64_t T, int k, int E) {
+bool dense_segments(int64_t T, int k, int E) {
   const int64_t slots = T * k;
-  const int64_t seg_max = slots < E ? slots : E;
-  return slots >= kGemmMinSlotsPerExpert * seg_max;
+  return slots >= kDenseSlotsPerExpert * (slots < E ? slots : E);
+}
+
+// Where the line lies (us a layer, decode kernels / GEMMs):
+//   token-tile shapes: Qwen3 at 4, 8, 16, 32 slots per expert 95 / 117, 128 to
+//     165 / 148, 173 / 166, 311 / 188; Mixtral at 4, 8, 16, 32 165 / 187,
+//     175 / 189, 309 / 232, 520 / 300.  The token-tile kernels read an
+//     expert's weights once per 16-position tile: about 8 slots per expert
+//     they are ahead only as long as no expert has more than 16.
+//   shapes of the K-split kernels (rows of H too long for a token tile's
+//     operand in LDS) with work for the chip: DeepSeek-V3 at 8 tokens (a
+//     quarter of its experts active) 316 / 342, at 1, 2, 4, 8 slots per expert
+//     873 / 806, 1196 / 1074, 1630 / 1347, 1951 / 1426.
+// With few GEMM items (few experts, short I) the K-split kernels fill the chip.
+bool gemm_regime(int64_t T, int64_t H, int64_t I, int k, int E, int has_shared) {
+  if (dense_segments(T, k, E)) return true;
+  if (lib_config().force_ksplit) return false;
+  const int64_t slots = T * k, experts = slots < E ? slots : E;
+  const int64_t Kq = ceil_div(H, kQuad), KqI = ceil_div(I, kQuad);
+  const int64_t lim = (int64_t)1 << 31;
+  if (T * Kq * 256 >= lim || I * Kq * 64 >= lim || H * KqI * 64 >= lim) return false;  // 32-bit offsets
+  if (gate_up_tile_regime(T, H, I, E, k, has_shared)) return slots >= 12 * experts;
+  return slots >= E && experts * ceil_div(I, kG2Waves * 16) >= 4 * (int64_t)device_cus();
 }
 
 // One launch: position blocks of BM times row blocks of `rows`, on the

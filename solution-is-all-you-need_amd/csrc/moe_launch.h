@@ -261,11 +261,13 @@ struct ExpertArgs {
   const float* topk_w;
   float* y;
 };
-// Prefill regime: when the average segment holds at least this many slots,
-// the expert stages run as grouped MFMA GEMMs (expert_gemm.hip) on fp16
-// operands; below it, as the grouped GEMV (expert_ffn.hip).
-constexpr int kGemmMinSlotsPerExpert = 64;
-bool gemm_regime(int64_t T, int k, int E);
+// Segments of at least this many slots on average always run as GEMMs; below
+// it a call is bound by the decode kernels' size limit, whichever kernels run.
+constexpr int kDenseSlotsPerExpert = 64;
+bool dense_segments(int64_t T, int k, int E);
+// Whether the expert stages run as grouped MFMA GEMMs (expert_gemm.hip) on
+// fp16 operands, or as the grouped GEMVs (expert_ffn.hip).
+bool gemm_regime(int64_t T, int64_t H, int64_t I, int k, int E, int has_shared);
 hipError_t launch_gemm_gate_up(const ExpertArgs& a, const Workspace& ws, hipStream_t stream);
 hipError_t launch_gemm_down(const ExpertArgs& a, const Workspace& ws, hipStream_t stream);
 
