@@ -200,7 +200,7 @@ size_t plan_workspace(int64_t T, int64_t H, int64_t I, int E, int k, int has_sha
                       Workspace* ws);
 
 // Router tiling: tokens per logits workgroup tile.
-int router_token_tile(int64_t T);
+int router_token_tile(int64_t T, int E);
 // Batches routed in two passes (approximate logits with an error bound, then
 // the exact logits of the candidates): bf16 x, T >= 128, E >= 16.  The
 // workspace holds their regions (approx, cand) whenever T and E qualify.

@@ -168,3 +168,20 @@ def test_systematic_bf16_ties(dev):
     for k in (1, 2):
         ridx = check(dev, xb, W, k)
         assert (ridx[:, 0] == 3).all()
+
+
+# (T, H, E): the split-K approximate kernels with one and two token tiles a
+# workgroup and the 64-token kernel (at most 64, at most 128 and more
+# 16-expert x 64-token blocks), both groupings of the exact kernel (at most 512
+# expert x 256-token blocks), ragged tokens and experts, and rows that end
+# inside a wave's first, second and fifth 128-wide chunk
+@pytest.mark.parametrize("T,H,E", [
+    (128, 32, 16), (129, 160, 17), (200, 672, 40), (500, 2016, 120),  # one tile
+    (321, 544, 250), (1000, 2048, 66),                                  # two
+    (577, 800, 256), (1100, 512, 120),                                  # 64 tokens
+])
+def test_split_kernels(dev, T, H, E):
+    rng, xb, W = base_inputs(T, H, E, seed=T + H)
+    W[E // 2] = W[0]  # an exact tie across expert tiles
+    W[1] = W[0] * np.float32(1 + 2 ** -22)
+    check(dev, xb, W, min(8, E))
