@@ -30,25 +30,30 @@
 // 1.2 PFLOP/s (gate/up) and 0.75 PFLOP/s (down, two MFMAs a product) here;
 // plain MFMAs reach 1.5.
 //
-// Two workgroups of four waves per CU.  A workgroup owns BM consecutive
-// positions of one expert segment and 4 x 2 row tiles of weights, so a CU
-// always holds two items that share no barrier: one's prologue (item lookup,
-// first copies), epilogue (SwiGLU, stores) and barrier waits run under the
-// other's MFMAs.  (One eight-wave workgroup per CU spent 28% of gate/up and
+// Two (gate/up) or three (down) workgroups of four waves per CU.  A workgroup
+// owns BM consecutive positions of one expert segment and 4 x 2 row tiles of
+// weights, so a CU holds items that share no barrier: one's prologue (item
+// lookup, first copies), epilogue (SwiGLU, stores) and barrier waits run under
+// another's MFMAs.  (One eight-wave workgroup per CU spent 28% of gate/up and
 // 36% of down outside the K loop at 4096 tokens: all eight waves were in the
-// prologue or the epilogue at the same time.)
+// prologue or the epilogue at the same time.)  Down's blocks of 64 positions
+// need half the accumulators, so three of its workgroups fit: 1417 -> 1226 us
+// at DeepSeek-V3 2048 tokens, 257 -> 241 at Qwen3 4096, against two with a
+// deeper ring (ahead only where the launch has one workgroup per CU: Mixtral
+// at 64 tokens 99 against 115).
 //
 // Operand ring.  Both operands come by direct-to-LDS loads, issued from inline
 // assembly (dma_b128_unseen) so that the compiler adds no waits of its own;
 // each wave copies its own weight tiles and a share of the A rows, waits for
 // its copies of the step about to be read, and one workgroup barrier per step
 // publishes them (and says that every wave has left the slot about to be
-// refilled).  A CU's 160 KB give each workgroup 75 KB of ring (RingCfg): with
-// few positions a step is a whole K quad of both operands and the ring is
-// three to five steps deep, which is what streams weights from HBM; at 80
-// positions and more a step is half a quad of A (three slots) and the weights
-// keep a ring of three quads.  A rows are stored with 16-byte unit s of row r
-// at s ^ a_swizzle(r): no ds_read_b128 of A has a bank conflict.
+// refilled).  A workgroup has 75 KB (gate/up) or 50 KB (down) of a CU's 160 KB
+// for its ring (RingCfg).  Gate/up up to 64 positions: a step is a whole K quad
+// of both operands and the ring is three to five steps deep, which is what
+// streams weights from HBM.  Above, and in down: a step is half a quad of A
+// (three slots, or two) and the weights keep a ring of quads (three, or two).
+// A rows are stored with 16-byte unit s of row r at s ^ a_swizzle(r): no
+// ds_read_b128 of A has a bank conflict.
 //
 // Tiling.  Every wave multiplies all BM positions with two weight row tiles of
 // its own, so each B operand feeds one MFMA (down: two) per 16-position tile
@@ -322,23 +327,32 @@ constexpr int kG2NB = 2;  // weight row tiles per wave in both kernels
 constexpr int kG2BNib = kG2Waves * kG2NB * kWave;          // nibbles: one 1 KiB unit row per operand
 constexpr int kG2BUnits = kG2BNib + kG2Waves * kG2NB * 8;  // and 128 B of scales per operand
 constexpr int kG2BLoads = 2 * kG2NB;                       // weight copies per wave per quad
-constexpr int kG2RingUnits = 4800;  // 75 KB: two workgroups and their tables in a CU's 160 KB
+// Ring of a workgroup: 75 KB for gate/up (two workgroups and their tables in a
+// CU's 160 KB), 50 KB for down (three; its blocks need fewer registers).
+template <int AW>
+constexpr int kG2RingUnits = AW == 1 ? 4800 : 3200;
+template <int AW>
+constexpr int kG2PerCu = AW == 1 ? 2 : 3;
 
 // The ring of a block whose leading VT 16-position tiles are multiplied
 // (16-byte units).
 template <int AW, int VT>
 struct RingCfg {
-  // a step is a quad of both operands (few positions), else half a quad of A
-  static constexpr bool kHalf = AW * VT > 4;
+  static constexpr int kRing = kG2RingUnits<AW>;
+  // a step is a quad of both operands (gate/up, few positions), else half a quad of A
+  static constexpr bool kHalf = AW == 2 || VT > 4;
   static constexpr int kUpr = (kHalf ? 8 : 16) * AW;  // units per A row per step
   static constexpr int kRpd = kWave / kUpr;           // A rows per copy
   // A copies per wave per step: only those that reach a multiplied tile
   static constexpr int kALoads = (16 * VT + kG2Waves * kRpd - 1) / (kG2Waves * kRpd);
   static constexpr int kAUnits = kALoads * kG2Waves * kWave;
-  // whole quads: slots of the ring; half quads: three A slots and three of B quads
+  // whole quads: slots of the ring
   static constexpr int kSlot = kAUnits + kG2BUnits;
-  static constexpr int kSlots = kG2RingUnits / kSlot > 5 ? 5 : kG2RingUnits / kSlot;
-  static_assert(kHalf ? 3 * kSlot <= kG2RingUnits : kSlots >= 3, "the ring fits");
+  static constexpr int kSlots = kRing / kSlot > 5 ? 5 : kRing / kSlot;
+  // half quads: A slots (halves) and B slots (quads)
+  static constexpr int kSlotsA = 3 * kAUnits + 2 * kG2BUnits <= kRing ? 3 : 2;
+  static constexpr int kSlotsB = kSlotsA == 3 && 3 * kSlot <= kRing ? 3 : 2;
+  static_assert(kHalf ? kSlotsA * kAUnits + kSlotsB * kG2BUnits <= kRing : kSlots >= 3, "the ring fits");
 };
 
 // Column swizzle of the A rows in LDS.  gfx950 serves a wave's ds_read_b128
@@ -556,31 +570,43 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmK& a, 
                                    a_lane, mask, acc);
     }
   } else {
-    // A in three slots of half a quad, two steps ahead; B in three slots of a
-    // quad, two quads ahead, refilled on even steps (before the step's A copies)
-    constexpr uint32_t kB0 = 3 * C::kAUnits;
+    // A in NA slots of half a quad, B in NQ slots of a quad, each refilled as
+    // far ahead as its slots allow, B on even steps
+    constexpr uint32_t NA = C::kSlotsA, NQ = C::kSlotsB;
+    constexpr uint32_t kB0 = NA * C::kAUnits;
     const uint32_t n_steps = (Kg + 1) / 2;
     copy_b(0, kB0);
-    if (Kq > 1) copy_b(1, kB0 + kG2BUnits);
+    if (NQ == 3 && Kq > 1) copy_b(1, kB0 + kG2BUnits);
     copy_a(0, 0);
-    if (n_steps > 1) copy_a(1, C::kAUnits);
+    if (NA == 3 && n_steps > 1) copy_a(1, C::kAUnits);
     uint32_t sa = 0, sb = 0;
     auto top = [&](uint32_t s, bool odd) {
       asm volatile("" ::: "memory");
-      // newer than step s's copies: step s + 1's A, and the weights copied before it
-      if (s + 1 >= n_steps) wait_vm_lgkm0<0>();
-      else if (odd && (s >> 1) + 2 < Kq) wait_vm_lgkm0<C::kALoads + kG2BLoads>();
-      else wait_vm_lgkm0<C::kALoads>();
+      if constexpr (NA == 3) {
+        // newer than this step's A: the next step's, and the weights copied before it
+        if (s + 1 >= n_steps) wait_vm_lgkm0<0>();
+        else if (odd && (s >> 1) + NQ - 1 < Kq) wait_vm_lgkm0<C::kALoads + kG2BLoads>();
+        else wait_vm_lgkm0<C::kALoads>();
+      } else {
+        // this step's A was copied a step ago, the weights after it
+        if (odd && (s >> 1) + NQ - 1 < Kq) wait_vm_lgkm0<kG2BLoads>();
+        else wait_vm_lgkm0<0>();
+      }
       __builtin_amdgcn_s_barrier();  // every copy of step s is in; step s - 1's slots are free
       asm volatile("" ::: "memory");
-      if (!odd && (s >> 1) + 2 < Kq) copy_b((s >> 1) + 2, kB0 + (sb == 0 ? 2u : sb - 1u) * kG2BUnits);
-      if (s + 2 < n_steps) copy_a(s + 2, (sa == 0 ? 2u : sa - 1u) * C::kAUnits);
+      auto refill_b = [&] {
+        if (!odd && (s >> 1) + NQ - 1 < Kq)
+          copy_b((s >> 1) + NQ - 1, kB0 + (sb == 0 ? NQ - 1 : sb - 1u) * kG2BUnits);
+      };
+      if constexpr (NA == 3) refill_b();
+      if (s + NA - 1 < n_steps) copy_a(s + NA - 1, (sa == 0 ? NA - 1 : sa - 1u) * C::kAUnits);
+      if constexpr (NA == 2) refill_b();
     };
     auto math = [&](auto ragged, bool odd) {
       const uint32_t ub = kB0 + sb * kG2BUnits;
       step_math<AW, VT, BMT, decltype(ragged)::value>(lds + sa * C::kAUnits, nib_of(ub), scale_of(ub), odd ? 2 : 0, 1,
                                                       a_lane, mask, acc);
-      sa = sa == 2 ? 0u : sa + 1u;
+      sa = sa == NA - 1 ? 0u : sa + 1u;
     };
     const uint32_t full = Kg / 2;  // steps with both groups
     uint32_t s = 0;
@@ -589,7 +615,7 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmK& a, 
       math(std::false_type(), false);
       top(s + 1, true);
       math(std::false_type(), true);
-      sb = sb == 2 ? 0u : sb + 1u;
+      sb = sb == NQ - 1 ? 0u : sb + 1u;
     }
     if (s < full) {
       top(s, false);
@@ -619,12 +645,12 @@ __device__ __attribute__((always_inline)) inline void gemm_tiles(int vt, Args&&.
   }
 }
 
-__global__ __launch_bounds__(kG2Waves * kWave, 2) void gemm_gate_up_kernel(GemmK a) {
+__global__ __launch_bounds__(kG2Waves * kWave, kG2PerCu<1>) void gemm_gate_up_kernel(GemmK a) {
   constexpr int BM = kGateUpBM;
   constexpr int TT = BM / 16;
   constexpr int kTiles = kG2Waves;  // row tiles of I per workgroup: half a quad of h,
   constexpr int kUr = 16;           // 16 units of 16 bytes per position
-  __shared__ u32x4 lds_a[kG2RingUnits];
+  __shared__ u32x4 lds_a[kG2RingUnits<1>];
   __shared__ int s_mb[kMaxExperts + 2];
   __shared__ uint32_t s_row[BM];
   __shared__ float s_un[BM];
@@ -727,13 +753,13 @@ __global__ __launch_bounds__(kG2Waves * kWave, 2) void gemm_gate_up_kernel(GemmK
   }
 }
 
-__global__ __launch_bounds__(kG2Waves * kWave, 2) void gemm_down_kernel(GemmK a) {
+__global__ __launch_bounds__(kG2Waves * kWave, kG2PerCu<2>) void gemm_down_kernel(GemmK a) {
   constexpr int BM = kDownBM;
   constexpr int TT = BM / 16;
   constexpr int NB = kG2NB;
   constexpr int kRows = kG2Waves * 16 * NB;  // rows of H per workgroup
-  static_assert(BM * kRows / 4 <= kG2RingUnits, "the epilogue's rows fit the ring");
-  __shared__ u32x4 lds_a[kG2RingUnits];
+  static_assert(BM * kRows / 4 <= kG2RingUnits<2>, "the epilogue's rows fit the ring");
+  __shared__ u32x4 lds_a[kG2RingUnits<2>];
   __shared__ int s_mb[kMaxExperts + 2];
   __shared__ uint32_t s_row[BM];
   __shared__ BlockPlan s_plan;

@@ -542,7 +542,9 @@ __device__ inline int tree_pair_of_lane(int lane) {
   return pair;
 }
 
-template <typename XT, int TT, int EW, int CB>
+// PREP16: the launch writes the GEMM regime's copy of x (its code would cost the
+// other launches registers).
+template <typename XT, int TT, int EW, int CB, bool PREP16>
 __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
   constexpr int P = TT * EW;
   static_assert((P & (P - 1)) == 0 && P <= 64, "pairs per wave must be a power of two <= 64");
@@ -600,7 +602,7 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
     }
     // the MFMA-ordered copy of x, its loads in flight with the first batch's
     if (c0 == 0 && a.prep_x) {
-      if (!a.prep_fp16) {
+      if constexpr (!PREP16) {
         prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
       } else {
         __shared__ uint32_t s_mx[4];
@@ -652,7 +654,7 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
     }
   }
 
-  if (a.prep_x && !a.prep_fp16 && blockIdx.x == 1 % gridDim.x && blockIdx.y == 0) {
+  if (!PREP16 && a.prep_x && blockIdx.x == 1 % gridDim.x && blockIdx.y == 0) {
     // all-zero activation row T, read by expert lanes past a segment
     for (int64_t i = threadIdx.x; i < a.Kq * 128; i += blockDim.x) a.xq[a.T * a.Kq * 128 + i] = 0;
     for (int64_t i = threadIdx.x; i < a.Kq * 4; i += blockDim.x) a.xs[a.T * a.Kq * 4 + i] = 0.0f;
@@ -1794,19 +1796,19 @@ int router_token_tile(int64_t T, int E) {
   return kBigTT;
 }
 
-template <typename XT>
+template <typename XT, bool PREP16>
 static hipError_t launch_logits_t(const RouteK& k, int TT, int n_ttiles, hipStream_t stream) {
   if (TT == 1) {
     dim3 grid((unsigned)ceil_div(k.E, 4 * 1), (unsigned)n_ttiles);
-    hipLaunchKernelGGL((route_logits_kernel<XT, 1, 1, 8>), grid, dim3(256), 0, stream, k);
+    hipLaunchKernelGGL((route_logits_kernel<XT, 1, 1, 8, PREP16>), grid, dim3(256), 0, stream, k);
   } else if (TT == 2) {
     dim3 grid((unsigned)ceil_div(k.E, 4 * 2), (unsigned)n_ttiles);
-    hipLaunchKernelGGL((route_logits_kernel<XT, 2, 2, 8>), grid, dim3(256), 0, stream, k);
+    hipLaunchKernelGGL((route_logits_kernel<XT, 2, 2, 8, PREP16>), grid, dim3(256), 0, stream, k);
   } else if (TT == 4) {
     // batches of four chunks: with eight the bf16 kernel needs 256 registers
     // (one wave a SIMD) and the 64-token route took 43.4 us, with four 203
     dim3 grid((unsigned)ceil_div(k.E, 4 * 2), (unsigned)n_ttiles);
-    hipLaunchKernelGGL((route_logits_kernel<XT, 4, 2, 4>), grid, dim3(256), 0, stream, k);
+    hipLaunchKernelGGL((route_logits_kernel<XT, 4, 2, 4, PREP16>), grid, dim3(256), 0, stream, k);
   } else {
     dim3 grid((unsigned)ceil_div(k.E, 4 * kBigEW), (unsigned)n_ttiles);
     hipLaunchKernelGGL((route_logits_big_kernel<XT, kBigTT, kBigEW>), grid, dim3(256), 0, stream, k);
@@ -1902,8 +1904,9 @@ hipError_t launch_route(const RouteArgs& r, const Workspace& ws, hipStream_t str
   k.perm_chunk = ceil_div(n_slots, perm_blocks(n_slots));
   hipError_t err = two_pass
                        ? launch_route_two_pass(k, ws, stream)
-                       : ((r.x_dtype == 0) ? launch_logits_t<uint16_t>(k, TT, n_ttiles, stream)
-                                           : launch_logits_t<float>(k, TT, n_ttiles, stream));
+                       : r.x_dtype != 0 ? launch_logits_t<float, false>(k, TT, n_ttiles, stream)
+                       : r.prep_fp16    ? launch_logits_t<uint16_t, true>(k, TT, n_ttiles, stream)
+                                        : launch_logits_t<uint16_t, false>(k, TT, n_ttiles, stream);
   if (err != hipSuccess) return err;
   // One wave per token, four tokens per workgroup, so selection is spread
   // over many CUs.  The permute runs in the select launch up to
