@@ -177,10 +177,15 @@ __device__ __attribute__((always_inline)) inline void block_permute(const int32_
   int nbits = 1;
   while ((1 << nbits) < E) ++nbits;
 
-  for (int i = tid; i < NW * kMaxExperts; i += blockDim.x) s_cnt[i / kMaxExperts][i % kMaxExperts] = 0;
+  // slot numbers stay under 2^30: 32-bit divisions (a 64-bit one is some
+  // hundred instructions, on the route's critical path)
+  const uint32_t n32 = (uint32_t)n;
+  const uint32_t chunk32 = ((n32 + (uint32_t)NW - 1) / (uint32_t)NW + kWave - 1) / kWave * kWave;
+  const int64_t chunk = chunk32;
+  const int NU = (int)((n32 + chunk32 - 1) / chunk32);  // waves that hold slots
+  for (int i = tid; i < NU * kMaxExperts; i += blockDim.x) s_cnt[i / kMaxExperts][i % kMaxExperts] = 0;
   lds_barrier();
 
-  const int64_t chunk = round_up(ceil_div(n, NW), kWave);
   const int64_t beg = w * chunk;
   const int64_t end = (beg + chunk < n) ? beg + chunk : n;
 
@@ -241,7 +246,7 @@ __device__ __attribute__((always_inline)) inline void block_permute(const int32_
     const int e = tid * kPer + i;
     int t = 0;
     if (e < E && tid * kPer < kMaxExperts) {
-      for (int ww = 0; ww < NW; ++ww) t += s_cnt[ww][e];
+      for (int ww = 0; ww < NU; ++ww) t += s_cnt[ww][e];
     }
     tot[i] = t;
     act[i] = (t > 0) ? 1 : 0;
@@ -277,7 +282,7 @@ __device__ __attribute__((always_inline)) inline void block_permute(const int32_
       }
       trun += (tot[i] + 15) / 16;
       int b = run;
-      for (int ww = 0; ww < NW; ++ww) {
+      for (int ww = 0; ww < NU; ++ww) {
         const int c = s_cnt[ww][e];
         s_cnt[ww][e] = b;  // becomes the running base of (expert, wave)
         b += c;
@@ -328,10 +333,10 @@ __device__ __attribute__((always_inline)) inline void block_permute(const int32_
       const int pos = s_cnt[w][e] + __popcll(below);
       sorted_slots[pos] = (int32_t)sl;
       slot_pos[sl] = pos;
-      if (seg_tok) seg_tok[pos] = (int32_t)(sl / k);
+      if (seg_tok) seg_tok[pos] = (int32_t)((uint32_t)sl / (uint32_t)k);
       if (tiles) {
         const int rel = pos - s_beg[e];
-        tiles[(int64_t)(s_tb[e] + rel / 16) * kTileWords + 4 + rel % 16] = (int32_t)(sl / k);
+        tiles[(int64_t)(s_tb[e] + rel / 16) * kTileWords + 4 + rel % 16] = (int32_t)((uint32_t)sl / (uint32_t)k);
       }
       // Every lane of the group has read the base before the leader bumps
       // it: LDS operations of one wave complete in program order, and the
@@ -667,22 +672,27 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
 // waves for up to 64 tokens, its selection handed to the permute in LDS,
 // measured slower than the hand-off: route 24.4 vs 19.2 us at 32 tokens,
 // 57 vs 39 us at 64 tokens of H 7168.)
+//
+// Up to kSingleSelectTokens tokens a launch that permutes is one workgroup with
+// a wave per token (WAVES = 8): the permute then needs no hand-off between
+// workgroups (a release, an atomic's round trip and an acquire).
 constexpr int kSelectWaves = 4;
+constexpr int kSingleSelectTokens = 8;
 constexpr int kFusedSelectBlocks = 16;
 
-template <int NV>
-__global__ __launch_bounds__(256) void route_select_kernel(RouteK a) {
-  __shared__ uint64_t s_ck[kSelectWaves][kMaxTopK];
-  __shared__ double s_cv[kSelectWaves][kMaxTopK];
-  __shared__ int s_ci[kSelectWaves][kMaxTopK];
-  __shared__ double s_val[kSelectWaves][kMaxTopK];
-  __shared__ double s_e[kSelectWaves][kMaxTopK];
-  __shared__ int s_idx[kSelectWaves][kMaxTopK];
-  __shared__ int s_sel[kSelectWaves * kMaxTopK];  // one workgroup: every token's selection, for the permute
+template <int NV, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void route_select_kernel(RouteK a) {
+  __shared__ uint64_t s_ck[WAVES][kMaxTopK];
+  __shared__ double s_cv[WAVES][kMaxTopK];
+  __shared__ int s_ci[WAVES][kMaxTopK];
+  __shared__ double s_val[WAVES][kMaxTopK];
+  __shared__ double s_e[WAVES][kMaxTopK];
+  __shared__ int s_idx[WAVES][kMaxTopK];
+  __shared__ int s_sel[WAVES * kMaxTopK];  // one workgroup: every token's selection, for the permute
   __shared__ int s_last;
   const int w = threadIdx.x / kWave;
   const int nw = blockDim.x / kWave;
-  const bool single = gridDim.x == 1 && a.T <= kSelectWaves;
+  const bool single = gridDim.x == 1 && a.T <= WAVES;
   const int lane = threadIdx.x % kWave;
   for (int64_t t = (int64_t)blockIdx.x * nw + w; t < a.T; t += (int64_t)gridDim.x * nw) {
     wave_topk<NV>(a, t, s_ck[w], s_cv[w], s_ci[w], s_val[w], s_idx[w], s_e[w], single ? s_sel : nullptr);
@@ -690,7 +700,7 @@ __global__ __launch_bounds__(256) void route_select_kernel(RouteK a) {
     // selection of slot j is in s_idx[j] (this wave's own LDS stores)
     if (a.perm_cnt && lane < a.k) {
       const int e = s_idx[w][lane];
-      if (e >= 0 && e < a.E) atomicAdd(a.perm_cnt + (int64_t)e * a.perm_nb + (t * a.k + lane) / a.perm_chunk, 1);
+      if (e >= 0 && e < a.E) atomicAdd(a.perm_cnt + (int64_t)e * a.perm_nb + (uint32_t)(t * a.k + lane) / (uint32_t)a.perm_chunk, 1);
     }
   }
   if (!a.do_permute) return;
@@ -1403,10 +1413,10 @@ __device__ __attribute__((always_inline)) inline void perm_wave_rounds(
           const int pos = cnt_w[e] + __popcll(below);
           sorted_slots[pos] = (int32_t)sl;
           slot_pos[sl] = pos;
-          if (seg_tok) seg_tok[pos] = (int32_t)(sl / k);
+          if (seg_tok) seg_tok[pos] = (int32_t)((uint32_t)sl / (uint32_t)k);
           if (tiles) {
             const int rel = pos - s_beg[e];
-            tiles[(int64_t)(s_tb[e] + rel / 16) * kTileWords + 4 + rel % 16] = (int32_t)(sl / k);
+            tiles[(int64_t)(s_tb[e] + rel / 16) * kTileWords + 4 + rel % 16] = (int32_t)((uint32_t)sl / (uint32_t)k);
           }
           // every lane of the group read the base before the leader bumps it
           if (below == 0) cnt_w[e] = cnt_w[e] + __popcll(m);
@@ -1887,7 +1897,8 @@ hipError_t launch_route(const RouteArgs& r, const Workspace& ws, hipStream_t str
   const bool want_tiles = r.do_permute && r.want_tiles;
   k.tiles = want_tiles ? ws.tiles : nullptr;
   k.n_tiles = want_tiles ? ws.n_tiles : nullptr;
-  const unsigned sel_blocks = (unsigned)ceil_div(r.T, kSelectWaves);
+  const bool one_select = r.do_permute && r.T <= kSingleSelectTokens;
+  const unsigned sel_blocks = one_select ? 1u : (unsigned)ceil_div(r.T, kSelectWaves);
   k.fuse_permute = (r.do_permute && sel_blocks > 1 && sel_blocks <= kFusedSelectBlocks) ? 1 : 0;
   k.counter = k.fuse_permute ? ws.counter : nullptr;
   const GemmItems items = gemm_items(ws, r.T, r.H);
@@ -1911,11 +1922,21 @@ hipError_t launch_route(const RouteArgs& r, const Workspace& ws, hipStream_t str
   // One wave per token, four tokens per workgroup, so selection is spread
   // over many CUs.  The permute runs in the select launch up to
   // kFusedSelectBlocks workgroups, in its own single-workgroup launch beyond.
-  const dim3 sb(kWave * kSelectWaves);
-  if (r.E <= 64) hipLaunchKernelGGL(route_select_kernel<1>, dim3(sel_blocks), sb, 0, stream, k);
-  else if (r.E <= 128) hipLaunchKernelGGL(route_select_kernel<2>, dim3(sel_blocks), sb, 0, stream, k);
-  else if (r.E <= 256) hipLaunchKernelGGL(route_select_kernel<4>, dim3(sel_blocks), sb, 0, stream, k);
-  else hipLaunchKernelGGL(route_select_kernel<8>, dim3(sel_blocks), sb, 0, stream, k);
+  // (a single workgroup has at least four waves: its permute's scan covers the
+  // experts with two per thread)
+  const dim3 sb(kWave * (unsigned)(one_select && r.T > kSelectWaves ? r.T : kSelectWaves));
+#define PMOE_SELECT(NV_)                                                                               \
+  do {                                                                                                 \
+    if (one_select && r.T > kSelectWaves)                                                              \
+      hipLaunchKernelGGL((route_select_kernel<NV_, kSingleSelectTokens>), dim3(1), sb, 0, stream, k);  \
+    else                                                                                               \
+      hipLaunchKernelGGL((route_select_kernel<NV_, kSelectWaves>), dim3(sel_blocks), sb, 0, stream, k); \
+  } while (0)
+  if (r.E <= 64) PMOE_SELECT(1);
+  else if (r.E <= 128) PMOE_SELECT(2);
+  else if (r.E <= 256) PMOE_SELECT(4);
+  else PMOE_SELECT(8);
+#undef PMOE_SELECT
   err = hipGetLastError();
   if (err != hipSuccess || !r.do_permute || sel_blocks == 1 || k.fuse_permute) return err;
   if (r.T * r.k >= kPermMultiSlots)
