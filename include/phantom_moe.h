@@ -185,6 +185,13 @@ PHANTOM_MOE_API int phantom_moe_route(const void* x, int x_dtype, const float* r
                       int64_t T, int64_t H, int E, int top_k, int score_mode, int32_t* topk_idx,
                       float* topk_w, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* phantom_moe_route with 64-bit indices, the type the reference module
+ * returns (tests/test_moe_routing.py:67), so a caller that needs them converts
+ * nothing. */
+PHANTOM_MOE_API int phantom_moe_route_i64(const void* x, int x_dtype, const float* router_w, const float* router_bias,
+                      int64_t T, int64_t H, int E, int top_k, int score_mode, int64_t* topk_idx,
+                      float* topk_w, void* workspace, size_t workspace_bytes, hipStream_t stream);
+
 /* Stable counting sort of the T*top_k (token, slot) pairs by expert.
  * expert_offsets [E+1]: exclusive prefix sum of per-expert counts;
  * sorted_slots [T*top_k]: slot ids s = t*top_k + j in (expert, s) order;

@@ -476,6 +476,39 @@ int run_forward(const ForwardCall& c, void* workspace, hipStream_t stream) {
   return launch_status(record_stage(4, stream), "profile event");
 }
 
+// Both route entry points; exactly one of topk_idx and topk_idx64 is the
+// caller's.  With 64-bit indices the 32-bit ones stay in the workspace (in the
+// permute's region, which a route alone does not use).
+int run_route(const void* x, int x_dtype, const float* router_w, const float* router_bias, int64_t T, int64_t H, int E,
+              int top_k, int score_mode, int32_t* topk_idx, int64_t* topk_idx64, float* topk_w, void* workspace,
+              size_t workspace_bytes, hipStream_t stream) {
+  if (int rc = check_route_shapes(x, x_dtype, router_w, T, H, E, top_k, score_mode)) return rc;
+  if ((!topk_idx && !topk_idx64) || !topk_w)
+    return fail(PHANTOM_MOE_EINVAL, "topk_idx and topk_w must be non-null");
+  const size_t need = pmoe::plan_workspace(T, H, 0, E, top_k, 0, nullptr, nullptr);
+  if (!workspace || workspace_bytes < need)
+    return fail(PHANTOM_MOE_EWORKSPACE, "workspace of %zu bytes required, %zu given", need,
+                workspace ? workspace_bytes : (size_t)0);
+  pmoe::Workspace ws;
+  pmoe::plan_workspace(T, H, 0, E, top_k, 0, workspace, &ws);
+  pmoe::RouteArgs r = {};
+  r.x = x;
+  r.x_dtype = x_dtype;
+  r.router_w = router_w;
+  r.router_bias = router_bias;
+  r.T = T;
+  r.H = H;
+  r.E = E;
+  r.k = top_k;
+  r.score_mode = score_mode;
+  r.topk_idx = topk_idx ? topk_idx : ws.sorted_slots;
+  r.topk_idx64 = topk_idx64;
+  r.topk_w = topk_w;
+  r.prep_x = false;
+  r.do_permute = false;
+  return launch_status(pmoe::launch_route(r, ws, stream), "route");
+}
+
 }  // namespace
 
 extern "C" {
@@ -656,29 +689,15 @@ int phantom_moe_workspace_status(void* workspace, size_t workspace_bytes, uint32
 int phantom_moe_route(const void* x, int x_dtype, const float* router_w, const float* router_bias,
                       int64_t T, int64_t H, int E, int top_k, int score_mode, int32_t* topk_idx,
                       float* topk_w, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  if (int rc = check_route_shapes(x, x_dtype, router_w, T, H, E, top_k, score_mode)) return rc;
-  if (!topk_idx || !topk_w) return fail(PHANTOM_MOE_EINVAL, "topk_idx and topk_w must be non-null");
-  const size_t need = pmoe::plan_workspace(T, H, 0, E, top_k, 0, nullptr, nullptr);
-  if (!workspace || workspace_bytes < need)
-    return fail(PHANTOM_MOE_EWORKSPACE, "workspace of %zu bytes required, %zu given", need,
-                workspace ? workspace_bytes : (size_t)0);
-  pmoe::Workspace ws;
-  pmoe::plan_workspace(T, H, 0, E, top_k, 0, workspace, &ws);
-  pmoe::RouteArgs r = {};
-  r.x = x;
-  r.x_dtype = x_dtype;
-  r.router_w = router_w;
-  r.router_bias = router_bias;
-  r.T = T;
-  r.H = H;
-  r.E = E;
-  r.k = top_k;
-  r.score_mode = score_mode;
-  r.topk_idx = topk_idx;
-  r.topk_w = topk_w;
-  r.prep_x = false;
-  r.do_permute = false;
-  return launch_status(pmoe::launch_route(r, ws, stream), "route");
+  return run_route(x, x_dtype, router_w, router_bias, T, H, E, top_k, score_mode, topk_idx, nullptr, topk_w,
+                   workspace, workspace_bytes, stream);
+}
+
+int phantom_moe_route_i64(const void* x, int x_dtype, const float* router_w, const float* router_bias,
+                          int64_t T, int64_t H, int E, int top_k, int score_mode, int64_t* topk_idx,
+                          float* topk_w, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  return run_route(x, x_dtype, router_w, router_bias, T, H, E, top_k, score_mode, nullptr, topk_idx, topk_w,
+                   workspace, workspace_bytes, stream);
 }
 
 int phantom_moe_permute(const int32_t* topk_idx, int64_t T, int top_k, int E, int32_t* expert_offsets,

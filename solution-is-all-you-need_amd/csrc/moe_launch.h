@@ -226,6 +226,7 @@ struct RouteArgs {
   int64_t T, H;
   int E, k, score_mode;
   int32_t* topk_idx;
+  int64_t* topk_idx64;  // optional 64-bit copy
   float* topk_w;
   bool prep_x;       // write ws.xq / ws.xs
   bool prep_fp16;    // ws.xq as scaled fp16 and ws.xs its inverse scale per token (GEMM regime) instead of bf16 and group sums

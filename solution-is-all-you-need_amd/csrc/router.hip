@@ -46,6 +46,7 @@ struct RouteK {
   const float* bias;
   int64_t T, H;
   int E, k, score_mode;
+  int64_t* idx64;  // optional 64-bit copy of topk_idx
   int32_t* topk_idx;
   float* topk_w;
   double* logits;
@@ -698,6 +699,7 @@ __global__ __launch_bounds__(WAVES * kWave) void route_select_kernel(RouteK a) {
     wave_topk<NV>(a, t, s_ck[w], s_cv[w], s_ci[w], s_val[w], s_idx[w], s_e[w], single ? s_sel : nullptr);
     // slot t k + j (j = lane) counted for the many-slot permute; the
     // selection of slot j is in s_idx[j] (this wave's own LDS stores)
+    if (a.idx64 && lane < a.k) a.idx64[t * a.k + lane] = s_idx[w][lane];
     if (a.perm_cnt && lane < a.k) {
       const int e = s_idx[w][lane];
       if (e >= 0 && e < a.E) atomicAdd(a.perm_cnt + (int64_t)e * a.perm_nb + (uint32_t)(t * a.k + lane) / (uint32_t)a.perm_chunk, 1);
@@ -1875,6 +1877,7 @@ hipError_t launch_route(const RouteArgs& r, const Workspace& ws, hipStream_t str
   k.score_mode = r.score_mode;
   k.topk_idx = r.topk_idx;
   k.topk_w = r.topk_w;
+  k.idx64 = r.topk_idx64;
   k.logits = ws.logits;
   const int TT = router_token_tile(r.T, r.E);
   const int n_ttiles = (int)ceil_div(r.T, TT);

@@ -46,6 +46,7 @@ SIGNATURES = {
     "phantom_moe_set_option": (_int, [_int, _int]),
     "phantom_moe_get_option": (_int, [_int, _vp]),
     "phantom_moe_route": (_int, [_vp, _int, _vp, _vp, _i64, _i64, _int, _int, _int, _vp, _vp, _vp, _sz, _vp]),
+    "phantom_moe_route_i64": (_int, [_vp, _int, _vp, _vp, _i64, _i64, _int, _int, _int, _vp, _vp, _vp, _sz, _vp]),
     "phantom_moe_permute": (_int, [_vp, _i64, _int, _int, _vp, _vp, _vp, _vp, _sz, _vp]),
     "phantom_moe_forward": (
         _int,

@@ -111,9 +111,31 @@ class MoEWeights:
         return sum(t.numel() * t.element_size() for t in ts)
 
 
-def route(x: torch.Tensor, router_weight: torch.Tensor, top_k: int, score="softmax", router_bias=None):
+# phantom_moe_workspace_bytes per shape (T, H, I, E, k, shared)
+_ws_bytes: dict = {}
+
+
+def _workspace_bytes(lib, shape: tuple) -> int:
+    nbytes = _ws_bytes.get(shape)
+    if nbytes is None:
+        if len(_ws_bytes) >= 4096:
+            _ws_bytes.clear()
+        nbytes = _ws_bytes[shape] = lib.phantom_moe_workspace_bytes(*shape)
+    return nbytes
+
+
+def _f32_like(t: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """t as the library reads it: fp32, contiguous, on x's device (t itself if it is)."""
+    if t.dtype == torch.float32 and t.device == x.device and t.is_contiguous():
+        return t
+    return t.detach().to(device=x.device, dtype=torch.float32).contiguous()
+
+
+def route(x: torch.Tensor, router_weight: torch.Tensor, top_k: int, score="softmax", router_bias=None,
+          index_dtype: torch.dtype = torch.int32):
     """Router only.  x [T, H] bf16 or fp32 (leading dims are flattened);
-    router_weight [E, H] fp32.  Returns (topk_w fp32 [T, k], topk_idx int32 [T, k])."""
+    router_weight [E, H] fp32.  Returns (topk_w fp32 [T, k], topk_idx [T, k] of
+    index_dtype, int32 or int64)."""
     _need_cuda(x, "x")
     lead = x.shape[:-1]
     H = x.shape[-1]
@@ -122,29 +144,29 @@ def route(x: torch.Tensor, router_weight: torch.Tensor, top_k: int, score="softm
         x2 = x2.float()  # exact widening
     if x2.dtype not in (torch.bfloat16, torch.float32):
         raise TypeError(f"x must be bf16, fp16 or fp32, got {x.dtype}")
+    if index_dtype not in (torch.int32, torch.int64):
+        raise TypeError(f"index_dtype must be int32 or int64, got {index_dtype}")
     x2 = x2.contiguous()
-    W = router_weight.detach().to(device=x.device, dtype=torch.float32).contiguous()
+    W = _f32_like(router_weight, x)
     E = W.shape[0]
     if W.shape != (E, H):
         raise ValueError(f"router_weight must be [E, {H}], got {tuple(W.shape)}")
-    b = None
-    if router_bias is not None:
-        b = router_bias.detach().to(device=x.device, dtype=torch.float32).contiguous()
+    b = None if router_bias is None else _f32_like(router_bias, x)
     T = x2.shape[0]
-    idx = torch.empty((T, top_k), dtype=torch.int32, device=x.device)
-    w = torch.empty((T, top_k), dtype=torch.float32, device=x.device)
+    idx = torch.empty((*lead, top_k), dtype=index_dtype, device=x.device)
+    w = torch.empty((*lead, top_k), dtype=torch.float32, device=x.device)
     if T == 0:  # an empty batch routes to empty outputs
-        return w.reshape(*lead, top_k), idx.reshape(*lead, top_k)
+        return w, idx
     lib = _lib.load()
-    nbytes = lib.phantom_moe_workspace_bytes(T, H, 0, E, top_k, 0)
-    ws = workspace(x.device, nbytes)
-    rc = lib.phantom_moe_route(
+    stream = _lib.stream_handle(x.device)
+    ws = workspace(x.device, _workspace_bytes(lib, (T, H, 0, E, top_k, 0)), stream)
+    fn = lib.phantom_moe_route if index_dtype == torch.int32 else lib.phantom_moe_route_i64
+    rc = fn(
         x2.data_ptr(), 0 if x2.dtype == torch.bfloat16 else 1, W.data_ptr(), None if b is None else b.data_ptr(),
-        T, H, E, top_k, _score_mode(score), idx.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(),
-        _lib.stream_handle(x.device),
+        T, H, E, top_k, _score_mode(score), idx.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), stream,
     )
     _lib.check(rc, "phantom_moe_route")
-    return w.reshape(*lead, top_k), idx.reshape(*lead, top_k)
+    return w, idx
 
 
 def permute(topk_idx: torch.Tensor, num_experts: int):
@@ -167,10 +189,6 @@ def permute(topk_idx: torch.Tensor, num_experts: int):
                                  ws.data_ptr(), ws.numel(), _lib.stream_handle(idx.device))
     _lib.check(rc, "phantom_moe_permute")
     return off, ss, sp
-
-
-# phantom_moe_workspace_bytes per forward shape (T, H, I, E, k, shared)
-_ws_bytes: dict = {}
 
 
 def moe_forward(x: torch.Tensor, router_weight: torch.Tensor, experts: MoEWeights, top_k: int,
@@ -209,10 +227,7 @@ def moe_forward(x: torch.Tensor, router_weight: torch.Tensor, experts: MoEWeight
     lib = _lib.load()
     _lib.check_status()  # a failure an earlier call left
     has_sh = experts.shared is not None
-    shape = (T, H, experts.I, E, top_k, int(has_sh))
-    nbytes = _ws_bytes.get(shape)
-    if nbytes is None:
-        nbytes = _ws_bytes[shape] = lib.phantom_moe_workspace_bytes(*shape)
+    nbytes = _workspace_bytes(lib, (T, H, experts.I, E, top_k, int(has_sh)))
     stream = _lib.stream_handle(x.device)
     ws = workspace(x.device, nbytes, stream)
     sh = [t.data_ptr() for t in experts.shared] if has_sh else [None] * 6

@@ -45,9 +45,9 @@ class PhantomTopKRouter(nn.Module):
             top_weights: softmax over the selected logits, [..., top_k], x.dtype
             top_indices: selected experts, [..., top_k], int64, descending logit
         """
-        if torch.is_grad_enabled() and (self.gate.weight.requires_grad or x.requires_grad):
+        gate = self.gate
+        if torch.is_grad_enabled() and (gate.weight.requires_grad or x.requires_grad):
             raise RuntimeError("PhantomTopKRouter has no backward: call it under torch.no_grad() "
                                "or set gate.weight.requires_grad_(False)")
-        w, idx = ops.route(x, self.gate.weight, self.top_k, "softmax",
-                           self.gate.bias if self.gate.bias is not None else None)
-        return w.to(x.dtype), idx.to(torch.int64)
+        w, idx = ops.route(x, gate.weight, self.top_k, "softmax", gate.bias, index_dtype=torch.int64)
+        return w.to(x.dtype), idx
