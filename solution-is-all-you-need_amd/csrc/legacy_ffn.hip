@@ -39,10 +39,10 @@ namespace pmoe {
 
 constexpr int kLgWaves = 4;         // waves per workgroup
 constexpr int kLgChunk = kWave * 8; // dot-product elements per lane pass: 8 per lane
-constexpr int kLgRowsPredict = 8;   // predictor rows per wave
+constexpr int kLgRowsPredict = 8;   // predictor rows per wave, from two batch rows on
 constexpr int kLgRowsFfn = 4;       // dense branch: neurons (gate and up rows) per wave
 constexpr int kLgRowsSparse = 2;    // sparse branch: list positions per wave
-constexpr int kLgRowsDown = 4;      // down rows per wave
+constexpr int kLgRowsDown = 4;      // down rows per wave, from two batch rows on
 constexpr int kLgCompactThreads = 1024;
 
 enum LgMode { kLgPredict = 0, kLgDense = 1, kLgSparse = 2 };
@@ -175,9 +175,8 @@ __device__ inline float lg_pick(const float (&acc)[NR][BT], int i) {
 }
 
 // Predictor: R consecutive neurons x BT batch rows per wave.
-template <int BT, bool VEC, int U>
+template <int R, int BT, bool VEC, int U>
 __global__ __launch_bounds__(kLgWaves* kWave) void lg_predict_kernel(LgRowsK p) {
-  constexpr int R = kLgRowsPredict;
   const int lane = threadIdx.x % kWave;
   const int64_t n0 = ((int64_t)blockIdx.x * kLgWaves + threadIdx.x / kWave) * R;
   const int64_t b0 = (int64_t)blockIdx.y * BT;
@@ -396,28 +395,39 @@ __global__ __launch_bounds__(kLgWaves* kWave) void lg_down_kernel(const uint16_t
   }
 }
 
-// Active neuron list of one batch row per workgroup, in increasing order.
+// Active neuron list of one batch row per workgroup, in increasing order:
+// 16 neurons per thread, one 16-byte load where the row allows it, so a row of
+// 14336 takes one pass of the loop (four loads of single bytes and four passes
+// took 7.0 us, this 5.4).
 __global__ __launch_bounds__(kLgCompactThreads) void lg_compact_kernel(const uint8_t* __restrict__ mask,
                                                                        int32_t* __restrict__ idx,
                                                                        int32_t* __restrict__ count,
                                                                        int64_t D_ffn) {
   constexpr int kWaves = kLgCompactThreads / kWave;
+  constexpr int kPer = 16;
   __shared__ int s_wave[kWaves];
   const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
   const uint8_t* m = mask + (int64_t)blockIdx.x * D_ffn;
   int32_t* out = idx + (int64_t)blockIdx.x * D_ffn;
+  const bool vec = (reinterpret_cast<uintptr_t>(m) & 15u) == 0;
   int64_t base = 0;
-  for (int64_t t0 = 0; t0 < D_ffn; t0 += 4 * kLgCompactThreads) {
-    const int64_t e0 = t0 + 4 * tid;
-    bool on[4];
-    int cnt = 0;
+  for (int64_t t0 = 0; t0 < D_ffn; t0 += kPer * kLgCompactThreads) {
+    const int64_t e0 = t0 + kPer * tid;
+    uint32_t bits = 0;  // bit j: neuron e0 + j is active
+    if (vec && e0 + kPer <= D_ffn) {
+      const uint4 v = *reinterpret_cast<const uint4*>(m + e0);
+      const uint32_t q[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t e = e0 + j;
-      const uint8_t v = m[e < D_ffn ? e : D_ffn - 1];
-      on[j] = e < D_ffn && v != 0;
-      cnt += on[j] ? 1 : 0;
+      for (int j = 0; j < kPer; ++j) bits |= ((q[j / 4] >> (8 * (j % 4))) & 0xffu) != 0 ? 1u << j : 0u;
+    } else {
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) {
+        const int64_t e = e0 + j;
+        const uint8_t v = m[e < D_ffn ? e : D_ffn - 1];
+        bits |= e < D_ffn && v != 0 ? 1u << j : 0u;
+      }
     }
+    const int cnt = __popc(bits);
     int incl = cnt;
 #pragma unroll
     for (int s = 1; s < kWave; s <<= 1) {
@@ -434,8 +444,8 @@ __global__ __launch_bounds__(kLgCompactThreads) void lg_compact_kernel(const uin
     }
     int64_t pos = base + before + incl - cnt;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (on[j]) out[pos++] = (int32_t)(e0 + j);
+    for (int j = 0; j < kPer; ++j)
+      if ((bits >> j) & 1u) out[pos++] = (int32_t)(e0 + j);
     base += total;
     __syncthreads();
   }
@@ -457,9 +467,13 @@ int batch_tile(int64_t B) { return B >= 8 ? 8 : (B >= 4 ? 4 : (B >= 2 ? 2 : 1));
 // Loads in flight per lane: U chunks x (rows + batch rows) x 16 bytes.
 template <int BT, bool VEC>
 hipError_t launch_predict_bt(const LgRowsK& p, hipStream_t s) {
-  constexpr int U = BT == 1 ? 2 : 1;
-  const dim3 grid((unsigned)ceil_div(p.D_ffn, (int64_t)kLgWaves * kLgRowsPredict), (unsigned)ceil_div(p.B, BT));
-  hipLaunchKernelGGL((lg_predict_kernel<BT, VEC, U>), grid, dim3(kLgWaves * kWave), 0, s, p);
+  // One batch row: nothing shares a row's load, so few rows and deep loads.
+  // At D 4096, D_ffn 14336 (us): 8 rows x 2 chunks 30.3 (448 workgroups on 256
+  // CUs), 4 x 4 24.3, 4 x 2 25.2, 2 x 4 23.7, 2 x 8 24.4.
+  constexpr int R = BT == 1 ? 2 : kLgRowsPredict;
+  constexpr int U = BT == 1 ? 4 : 1;
+  const dim3 grid((unsigned)ceil_div(p.D_ffn, (int64_t)kLgWaves * R), (unsigned)ceil_div(p.B, BT));
+  hipLaunchKernelGGL((lg_predict_kernel<R, BT, VEC, U>), grid, dim3(kLgWaves * kWave), 0, s, p);
   return hipGetLastError();
 }
 
@@ -483,9 +497,12 @@ hipError_t launch_ffn_rows(const LgRowsK& p, hipStream_t s) {
 template <int MODE, int BT, bool VEC>
 hipError_t launch_down_bt(const uint16_t* act, const int32_t* mult, const uint16_t* wd, uint16_t* y, int64_t B,
                           int64_t D, int64_t D_ffn, hipStream_t s) {
-  constexpr int U = BT == 1 ? 2 : 1;
-  const dim3 grid((unsigned)ceil_div(D, (int64_t)kLgWaves * kLgRowsDown), (unsigned)ceil_div(B, BT));
-  hipLaunchKernelGGL((lg_down_kernel<MODE, kLgRowsDown, BT, VEC, U>), grid, dim3(kLgWaves * kWave), 0, s, act, mult,
+  // One batch row, as in the predictor (us): 4 rows x 2 chunks 26.9 (four waves
+  // a CU), 4 x 4 28.2, 2 x 4 24.4, 2 x 8 26.7, 1 x 4 29.5, 1 x 8 33.1.
+  constexpr int R = BT == 1 ? 2 : kLgRowsDown;
+  constexpr int U = BT == 1 ? 4 : 1;
+  const dim3 grid((unsigned)ceil_div(D, (int64_t)kLgWaves * R), (unsigned)ceil_div(B, BT));
+  hipLaunchKernelGGL((lg_down_kernel<MODE, R, BT, VEC, U>), grid, dim3(kLgWaves * kWave), 0, s, act, mult,
                      wd, y, B, D, D_ffn);
   return hipGetLastError();
 }

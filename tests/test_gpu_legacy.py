@@ -272,3 +272,19 @@ def test_calibrate_errors(dev):
         legacy.calibrate_sparsity_gate(x, torch.zeros((3, 8), dtype=torch.float32, device=dev))
     with pytest.raises(RuntimeError, match="float32"):
         legacy.calibrate_sparsity_gate(x.half(), torch.zeros((4, 8), dtype=torch.float32, device=dev))
+
+
+@pytest.mark.parametrize("D_ffn", [1, 15, 16, 17, 1024, 16384, 16385, 20000])
+def test_compaction_edges(dev, D_ffn):
+    """Row lengths around the 16 neurons a thread takes and the 16384 of a pass,
+    in rows that start on and off a 16-byte boundary: indices increasing and
+    complete."""
+    B, D = 3, 8
+    g = torch.Generator(device=dev).manual_seed(D_ffn)
+    x = torch.randn(B, D, generator=g, device=dev).half()
+    w = torch.randn(D_ffn, D, generator=g, device=dev).half()
+    mask, idx, cnt, _, _ = legacy.predict_active_neurons(x, w, None)
+    for b in range(B):
+        want = mask[b].nonzero().flatten().int()
+        assert int(cnt[b]) == want.numel()
+        assert torch.equal(idx[b, :want.numel()], want)
