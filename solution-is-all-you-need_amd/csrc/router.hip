@@ -46,7 +46,6 @@ struct RouteK {
   const float* bias;
   int64_t T, H;
   int E, k, score_mode;
-  int64_t* idx64;  // optional 64-bit copy of topk_idx
   int32_t* topk_idx;
   float* topk_w;
   double* logits;
@@ -70,8 +69,6 @@ struct RouteK {
   int32_t* tiles;    // token tiles (see kTileWords), or null
   int32_t* n_tiles;
   int32_t* counter;  // select workgroups finished (fused permute); zeroed by the logits launch
-  int32_t* items;  // the GEMM regime's 16 item counters, items_stride words apart, which the logits launch clears; or null
-  int items_stride;
   int fuse_permute;
   // many-slot permute: the select launch counts each slot into
   // perm_cnt[e * perm_nb + slot / perm_chunk] (zeroed by the first route
@@ -79,6 +76,9 @@ struct RouteK {
   int32_t* perm_cnt;
   int64_t perm_chunk;
   int perm_nb;
+  int64_t* idx64;  // optional 64-bit copy of topk_idx
+  int32_t* items;  // the GEMM regime's 16 item counters, items_stride words apart, which the logits launch clears; or null
+  int items_stride;
 };
 
 template <typename XT>
@@ -559,8 +559,12 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
   const int64_t t0 = (int64_t)blockIdx.y * TT;
   const int e0 = blockIdx.x * (4 * EW) + w * EW;
   const XT* x = static_cast<const XT*>(a.x);
+  // read with the first kernel arguments: left to where it is used, its scalar
+  // load is one more round trip before the weights' (0.5 us of 5.8)
+  int prep_x = a.prep_x;
+  asm volatile("" : "+s"(prep_x));
   if (a.counter && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.counter = 0;
-  if (a.items && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 16) a.items[threadIdx.x * a.items_stride] = 0;
+  if (PREP16 && a.items && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 16) a.items[threadIdx.x * a.items_stride] = 0;
   // The bias of the expert this lane may write, fetched ahead of the GEMV.
   float bias_e = 0.0f;
   if (a.bias) {
@@ -607,7 +611,7 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
       }
     }
     // the MFMA-ordered copy of x, its loads in flight with the first batch's
-    if (c0 == 0 && a.prep_x) {
+    if (c0 == 0 && prep_x) {
       if constexpr (!PREP16) {
         prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
       } else {
@@ -660,7 +664,7 @@ __global__ __launch_bounds__(256) void route_logits_kernel(RouteK a) {
     }
   }
 
-  if (!PREP16 && a.prep_x && blockIdx.x == 1 % gridDim.x && blockIdx.y == 0) {
+  if (!PREP16 && prep_x && blockIdx.x == 1 % gridDim.x && blockIdx.y == 0) {
     // all-zero activation row T, read by expert lanes past a segment
     for (int64_t i = threadIdx.x; i < a.Kq * 128; i += blockDim.x) a.xq[a.T * a.Kq * 128 + i] = 0;
     for (int64_t i = threadIdx.x; i < a.Kq * 4; i += blockDim.x) a.xs[a.T * a.Kq * 4 + i] = 0.0f;
@@ -869,8 +873,8 @@ __global__ __launch_bounds__(256) void route_logits_big_kernel(RouteK a) {
 // For prefill batches the fixed-order fp64 logits of every (token, expert)
 // pair cost 100 us at 4096 tokens of H 2048, E 128 -- while only the top k
 // of each token, and the experts near the k-th, decide anything.  So:
-//   route_approx_kernel: L~ = x . (w_hi + w_lo) on the matrix cores for every
-//     pair, with w_hi = bf16(w) and w_lo = bf16(w - w_hi) (both rounded to
+//   route_approx_kernel (or, for fewer tokens, route_approx_split_kernel):
+//     L~ = x . (w_hi + w_lo) on the matrix cores for every pair, with w_hi = bf16(w) and w_lo = bf16(w - w_hi) (both rounded to
 //     nearest), plus the norms |x_t| and |w_e|;
 //   route_candidates_kernel (one wave per token; four more waves per
 //     workgroup write the GEMM's copy of x meanwhile): the error bound
@@ -879,8 +883,8 @@ __global__ __launch_bounds__(256) void route_logits_big_kernel(RouteK a) {
 //     (a superset of the exact top k: any expert below that has k others
 //     strictly above it); the others' logits are set to -inf;
 //   route_exact_kernel (per expert and block of tokens): the fixed-order
-//     fp64 logits (contract above) of the candidate pairs, 16 tokens per wave
-//     so each lane's slice of the weight row is loaded once per 16 pairs;
+//     fp64 logits (contract above) of the candidate pairs, 4 or 16 tokens per
+//     wave so each lane's slice of the weight row is loaded once for them;
 //   route_select_kernel: the exact selection and weights, unchanged.
 // The bound.  Rounding: w - w_hi is exact in fp32, so |w - w_hi - w_lo| <=
 // 2^-8 |w - w_hi| <= 2^-16 |w| (an 8-bit significand rounds to within 2^-8
