@@ -653,7 +653,7 @@ __global__ __launch_bounds__(kG2Waves * kWave, kG2PerCu<1>) void gemm_gate_up_ke
   __shared__ u32x4 lds_a[kG2RingUnits<1>];
   __shared__ int s_mb[kMaxExperts + 2];
   __shared__ uint32_t s_row[BM];
-  __shared__ float s_un[BM];
+  __shared__ __align__(16) float s_un[BM];  // read as float4
   __shared__ BlockPlan s_plan;
   __shared__ int s_first[9], s_item;
   const int lane = threadIdx.x % kWave;
