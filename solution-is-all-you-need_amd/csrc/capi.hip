@@ -383,6 +383,12 @@ int check_forward(ForwardCall& c) {
   // most T positions of I as fp16 hi and lo) through a 32-bit buffer resource
   if (!pmoe::dense_segments(c.T, c.top_k, c.E) && c.T * ((c.I + 127) / 128) * 512 >= ((int64_t)1 << 31))
     return fail(PHANTOM_MOE_EUNSUPPORTED, "T*I too large for the decode regime (one segment's down operand above 2 GiB)");
+  // the GEMMs address the copy of x, whose rows an item gathers by token, and
+  // one expert's nibbles with 32-bit offsets (below 64 positions per expert
+  // gemm_regime leaves larger ones to the decode kernels)
+  const int64_t Kq = (c.H + 127) / 128, KqI = (c.I + 127) / 128, gib4 = (int64_t)1 << 32;
+  if (pmoe::dense_segments(c.T, c.top_k, c.E) && (c.T * Kq * 256 >= gib4 || c.I * Kq * 64 >= gib4 || c.H * KqI * 64 >= gib4))
+    return fail(PHANTOM_MOE_EUNSUPPORTED, "T*H or H*I too large for the GEMMs (the copy of x or one expert's matrix at 4 GiB)");
   return 0;
 }
 

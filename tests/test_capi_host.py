@@ -166,6 +166,16 @@ def _forward(**kw):
         # decode regime (under 64 positions per expert) with one segment's
         # down operand above 2 GiB
         (dict(T=32000, I=16896, E=512, k=1), EUNSUPPORTED),
+        # the GEMMs (64 positions per expert or more): the copy of x, or one
+        # expert's nibbles, at 4 GiB (the sizes just below pass on to the
+        # workspace check)
+        (dict(T=1 << 20, H=2048, E=16, k=1), EUNSUPPORTED),
+        (dict(T=(1 << 20) - 1, H=2048, E=16, k=1), EWORKSPACE),
+        (dict(T=1 << 24, H=96, E=16, k=2), EUNSUPPORTED),
+        (dict(T=64, H=1 << 16, I=1 << 17, E=1, k=1), EUNSUPPORTED),
+        (dict(T=64, H=1 << 16, I=(1 << 17) - 128, E=1, k=1), EWORKSPACE),
+        (dict(T=64, H=1 << 17, I=1 << 16, E=1, k=1), EUNSUPPORTED),
+        (dict(T=64, H=(1 << 17) - 32, I=1 << 16, E=1, k=1), EUNSUPPORTED),  # quads are padded
     ],
 )
 def test_forward_validation(kw, code):
