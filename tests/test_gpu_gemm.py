@@ -57,6 +57,50 @@ def test_gemm_edges(dev, shape):
     run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg))
 
 
+# Launches with fewer position blocks than the 8 item ranges, whose ranges are
+# cut between row blocks: 1, 3, 6 and 7 blocks (with the shared expert's), 8 and
+# 9 just past that line; 17 row blocks of I and 10 of H, the last ones ragged
+@pytest.mark.parametrize("shape", [(64, 1184, 1056, 1, 1, False), (192, 1184, 1056, 3, 1, False),
+                                   (70, 1184, 1056, 5, 5, True), (64, 1184, 1056, 7, 7, False),
+                                   (64, 1184, 1056, 8, 8, False), (64, 1184, 1056, 8, 8, True)],
+                         ids=lambda s: "-".join(str(int(v)) for v in s))
+def test_few_blocks(dev, shape):
+    T, H, I, E, k, shared = shape
+    cfg = synth.MoEConfig("few", H, I, E, k, T, shared=shared)
+    run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg))
+
+
+def test_one_block_uses_every_xcd(dev):
+    """One position block runs on all eight XCDs: its layer takes well under the
+    time of eight such blocks (one per XCD), which is what it took when a range
+    held whole blocks only."""
+    ms = []
+    for E in (1, 8):
+        cfg = synth.MoEConfig("spread", 4096, 8192, E, 1, 64 * E)
+        dl = synth.device_layer(cfg, dev)
+        ex = phantom_moe.MoEWeights.from_q4_0(dl.gate, dl.up, dl.down, cfg.H, cfg.I, cfg.E)
+        x = to_bf16_tensor(synth.activations(cfg.T, cfg.H), dev)
+        W = torch.zeros_like(dl.router_w)
+        W[:, :E] = 1000 * torch.eye(E, device=dev)
+        x[:, :E] = torch.eye(E, device=dev, dtype=x.dtype).repeat(64, 1)  # 64 tokens an expert
+
+        def call():
+            return phantom_moe.moe_forward(x, W, ex, 1, return_routing=True)
+
+        assert torch.bincount(call()[2].flatten().long(), minlength=E).tolist() == [64] * E
+        best = 1e9
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(4):
+                call()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        ms.append(best)
+    assert ms[0] < 0.7 * ms[1], ms
+
+
 # Just on either side of the line between the decode kernels and the GEMMs
 # below 64 slots per expert, for a shape of the token-tile kernels (12 slots
 # per expert) and one whose rows of H are too long for them (1 slot per expert)
