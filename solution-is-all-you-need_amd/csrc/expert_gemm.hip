@@ -216,10 +216,13 @@ __device__ inline int segment_of_block(const int* s_mb, int n_act, int mb) {
 // about once.  (Blocks dealt round-robin over the XCDs put the 2-3 blocks of
 // a segment on different XCDs, each streaming the segment's weights.)  Fewer
 // blocks than XCDs are cut between their row blocks instead, or some XCDs would
-// have no items: one block of 64 positions at H 2048, I 1024 134 -> 53 us a
-// layer, four experts at 64 tokens of H 2048, I 2048 90 -> 60.  (From 8 blocks
-// on that cut is no better, and splits segments of several blocks: Mixtral at
-// 256 tokens 421 -> 459 us.)
+// have no items (one block of 64 positions at H 2048, I 1024 134 -> 53 us a
+// layer, four experts at 96 tokens of H 2048, I 2048 106 -> 68), and so are 9 to
+// 15 blocks, of which some XCDs would have two and some one (nine experts and
+// the shared one at 33 tokens of H 5120, I 8192 339 -> 238; at 150 tokens of H
+// 2048, I 2048 92 -> 68).  In down only where no segment has two blocks: cut
+// apart, their XCDs would both stream its weights (Mixtral at 256 tokens 399
+// -> 433 us).
 //
 // Items are drawn, not dealt: a workgroup starts with item l of its XCD's
 // range and then draws from the range's counter, and from the other ranges'
@@ -278,15 +281,18 @@ struct ItemQueue {
 
 // s_first: [9] ints of LDS.  Item counts stay far below 2^31: an item writes
 // 32 KB of workspace.
-__device__ inline ItemQueue item_queue(int32_t* next, int stride, int n_mb, int n_nb, int* s_first) {
+// by_segment: two blocks of a segment should share an XCD.
+__device__ inline ItemQueue item_queue(int32_t* next, int stride, BlockPlan plan, bool by_segment, int n_nb,
+                                       int* s_first) {
   ItemQueue q;
   q.next = next;
   q.stride = stride;
   q.first = s_first;
   q.nx = gridDim.x < 8 ? (int)gridDim.x : 8;
   q.x0 = (int)(blockIdx.x % q.nx);
-  const int xr = (int)threadIdx.x;
-  if (xr <= q.nx) s_first[xr] = n_mb < q.nx ? n_mb * n_nb * xr / q.nx : n_mb * xr / q.nx * n_nb;
+  const int n_mb = plan.n_mb, xr = (int)threadIdx.x;
+  const bool uneven = n_mb < q.nx || (n_mb < 2 * q.nx && n_mb != q.nx && !(by_segment && n_mb > plan.n_act));
+  if (xr <= q.nx) s_first[xr] = uneven ? n_mb * n_nb * xr / q.nx : n_mb * xr / q.nx * n_nb;
   lds_barrier();
   const int f0 = __builtin_amdgcn_readfirstlane(s_first[q.x0]);
   q.item = f0 + (int)blockIdx.x / q.nx;
@@ -670,7 +676,7 @@ __global__ __launch_bounds__(kG2Waves * kWave, kG2PerCu<1>) void gemm_gate_up_ke
   const BlockPlan plan = plan_blocks<BM>(a.seg, s_mb, &s_plan);
   const int64_t n_tiles = a.N / kRowTile;
   const int n_nb = (int)ceil_div(n_tiles, kTiles);
-  ItemQueue queue = item_queue(a.items, a.items_stride, plan.n_mb, n_nb, s_first);
+  ItemQueue queue = item_queue(a.items, a.items_stride, plan, false, n_nb, s_first);
   const uint32_t nib_bytes = (uint32_t)(a.N * a.Kq * 64), sc_bytes = (uint32_t)(a.N * a.Kq * 8);
   // positions past the segment repeat its last row (computed, not stored)
   auto token_of = [&](const TileCoord& t) {
@@ -777,7 +783,7 @@ __global__ __launch_bounds__(kG2Waves * kWave, kG2PerCu<2>) void gemm_down_kerne
   const BlockPlan plan = plan_blocks<BM>(a.seg, s_mb, &s_plan);
   const int n_nb = (int)ceil_div(a.N, kRows);
   const int64_t n_tiles = a.N / kRowTile;
-  ItemQueue queue = item_queue(a.items, a.items_stride, plan.n_mb, n_nb, s_first);
+  ItemQueue queue = item_queue(a.items, a.items_stride, plan, true, n_nb, s_first);
   const uint32_t nib_bytes = (uint32_t)(a.N * a.Kq * 64), sc_bytes = (uint32_t)(a.N * a.Kq * 8);
   queue.next_item(&s_item);
   lds_barrier();

@@ -57,12 +57,14 @@ def test_gemm_edges(dev, shape):
     run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg))
 
 
-# Launches with fewer position blocks than the 8 item ranges, whose ranges are
-# cut between row blocks: 1, 3, 6 and 7 blocks (with the shared expert's), 8 and
-# 9 just past that line; 17 row blocks of I and 10 of H, the last ones ragged
+# Launches with few position blocks, whose item ranges are cut between row
+# blocks unless they are 8 or 16: 1, 3, 6, 7, 9 and 15 blocks in gate/up (with
+# the shared expert's); in down also 6 segments of two blocks, which stay whole;
+# 17 row blocks of I and 10 of H, the last ones ragged
 @pytest.mark.parametrize("shape", [(64, 1184, 1056, 1, 1, False), (192, 1184, 1056, 3, 1, False),
                                    (70, 1184, 1056, 5, 5, True), (64, 1184, 1056, 7, 7, False),
-                                   (64, 1184, 1056, 8, 8, False), (64, 1184, 1056, 8, 8, True)],
+                                   (64, 1184, 1056, 8, 8, False), (64, 1184, 1056, 8, 8, True),
+                                   (64, 416, 1056, 15, 15, False), (64, 416, 1056, 16, 16, False)],
                          ids=lambda s: "-".join(str(int(v)) for v in s))
 def test_few_blocks(dev, shape):
     T, H, I, E, k, shared = shape
