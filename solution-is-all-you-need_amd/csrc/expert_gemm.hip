@@ -851,26 +851,50 @@ bool dense_segments(int64_t T, int k, int E) {
   return slots >= kDenseSlotsPerExpert * (slots < E ? slots : E);
 }
 
-// Where the line lies (us a layer, decode kernels / GEMMs):
-//   token-tile shapes: Qwen3 at 4, 8, 16, 32 slots per expert 95 / 117, 128 to
-//     165 / 148, 173 / 166, 311 / 188; Mixtral at 4, 8, 16, 32 165 / 187,
-//     175 / 189, 309 / 232, 520 / 300.  The token-tile kernels read an
-//     expert's weights once per 16-position tile: about 8 slots per expert
-//     they are ahead only as long as no expert has more than 16.
+// Where the lines lie below 64 slots per expert: drawn so that a call is not
+// slower than on the decode kernels, over 1648 timed calls of 428 shapes (H 256
+// to 7168, I 128 to 14336, 4 to 256 experts, 1 to 1024 tokens); three are, by 6
+// to 8%, and none of 419 others by more than 3%.  (With a line at 12 slots per
+// expert alone, 149 of the first 1265 were, by up to 63%.)  Us a layer, decode
+// kernels / GEMMs:
+//   token-tile shapes, positions.  Those kernels read an expert's weights once
+//     per 16-position tile, so they are ahead as long as few experts have more
+//     than 16 positions: Qwen3 at 8, 12, 16, 32 slots per expert 152 / 129,
+//     157 / 135, 162 / 143, 296 / 168; Mixtral at 8, 12, 14, 16, 32 171 / 208,
+//     203 / 215, 281 / 248, 310 / 247, 512 / 319.  The second tile comes from
+//     cache where weights are few: E 141, H 3200, I 416 210 / 237 at 13, E 16,
+//     H 256, I 2048 41 / 47 at 12.
+//   token-tile shapes, positions x I.  A GEMM item is one workgroup's chain
+//     through K, so a launch needs items for the chip: E 10, H 2048, I 1024
+//     57 / 66 at 40 slots per expert (0.4 M), E 16, H 2048, I 1024 55 / 51 at 24
+//     (0.4 M) and 79 / 70 at 32 (0.5 M).  Where the K-split kernel would run
+//     down (short H), it takes longer for many positions, and the GEMMs are
+//     ahead sooner: E 20, H 512, I 768 60 / 51 at 32 slots per expert (0.5 M),
+//     most of all for a shared expert, one segment of all tokens: E 25, H 320,
+//     I 192 at 342 tokens 99 / 47 (0.19 M), E 26, H 352, I 448 at 201 78 / 50
+//     (0.26 M).
 //   shapes of the K-split kernels (rows of H too long for a token tile's
-//     operand in LDS) with work for the chip: DeepSeek-V3 at 8 tokens (a
-//     quarter of its experts active) 316 / 342, at 1, 2, 4, 8 slots per expert
-//     873 / 806, 1196 / 1074, 1630 / 1347, 1951 / 1426.
-// With few GEMM items (few experts, short I) the K-split kernels fill the chip.
+//     operand in LDS): DeepSeek-V3 at 1, 2, 4, 8 slots per expert 833 / 765,
+//     1189 / 1078, 1452 / 1298, 1904 / 1397.  Few tokens or short I again: H
+//     5120, E 160, I 448 173 / 183 at 64 tokens (0.23 M), H 7168, E 128, I 768
+//     181 / 214 at 32 tokens (0.10 M); H 5376, E 128, I 1024 and a shared expert
+//     305 / 238 at 48 (0.25 M).
 bool gemm_regime(int64_t T, int64_t H, int64_t I, int k, int E, int has_shared) {
   if (dense_segments(T, k, E)) return true;
   if (lib_config().force_ksplit) return false;
   const int64_t slots = T * k, experts = slots < E ? slots : E;
+  const int64_t work = (slots + (has_shared ? T : 0)) * I / 1024;
   const int64_t Kq = ceil_div(H, kQuad), KqI = ceil_div(I, kQuad);
   const int64_t lim = (int64_t)1 << 31;
   if (T * Kq * 256 >= lim || I * Kq * 64 >= lim || H * KqI * 64 >= lim) return false;  // 32-bit offsets
-  if (gate_up_tile_regime(T, H, I, E, k, has_shared)) return slots >= 12 * experts;
-  return slots >= E && experts * ceil_div(I, kG2Waves * 16) >= 4 * (int64_t)device_cus();
+  if (gate_up_tile_regime(T, H, I, E, k, has_shared)) {
+    const bool down_tile = down_tile_regime(T, H, I, E, k, has_shared);
+    const bool long_down = !down_tile && has_shared && T >= 64;
+    const int line = experts >= 16 && I >= 512 && work >= 512 ? 12 : (I >= 512 || long_down ? 14 : 16);
+    return slots >= line * experts && work >= (down_tile ? 512 : (long_down ? 160 : 320));
+  }
+  return slots >= E && slots + (has_shared ? T : 0) >= 64 && work >= 225 &&
+         experts * ceil_div(I, kG2Waves * 16) >= 4 * (int64_t)device_cus();
 }
 
 // One launch: position blocks of BM times row blocks of `rows`, on the

@@ -182,6 +182,52 @@ def test_forward_validation(kw, code):
     assert _forward(**kw) == code
 
 
+# (T, H, I, E, k, shared) -> whether the GEMMs run: both sides of each line of
+# gemm_regime (device attributes default to 256 CUs where there is no GPU)
+@pytest.mark.parametrize("shape,gemm", [
+    # token-tile shapes: 12 slots per expert from 16 experts of I 512 and
+    # 512 * 1024 positions x I on
+    ((191, 2048, 768, 128, 8, 0), False),
+    ((192, 2048, 768, 128, 8, 0), True),
+    ((96, 256, 2048, 16, 2, 0), False),
+    ((112, 256, 2048, 16, 2, 0), True),
+    # 14 slots for few experts, 16 for short I
+    ((55, 4096, 14336, 8, 2, 0), False),
+    ((56, 4096, 14336, 8, 2, 0), True),
+    ((918, 3200, 416, 141, 2, 1), False),
+    ((563, 3200, 416, 141, 4, 1), False),
+    ((564, 3200, 416, 141, 4, 1), True),
+    # and positions x I: 512 * 1024, 320 * 1024 where the K-split kernel would
+    # run down, 160 * 1024 where that has 64 positions of a shared expert
+    ((200, 2048, 1024, 10, 2, 0), False),
+    ((256, 2048, 1024, 10, 2, 0), True),
+    ((79, 1024, 2048, 8, 2, 0), False),
+    ((80, 1024, 2048, 8, 2, 0), True),
+    ((48, 2048, 2048, 4, 2, 0), False),
+    ((146, 320, 224, 32, 4, 1), False),
+    ((147, 320, 224, 32, 4, 1), True),
+    ((63, 320, 512, 16, 4, 1), False),
+    ((64, 320, 512, 16, 4, 1), True),
+    # K-split shapes: one slot per expert, 64 positions, 225 * 1024 positions x I
+    ((16, 5120, 2048, 32, 4, 0), False),
+    ((32, 5120, 2048, 32, 4, 0), True),
+    ((15, 5120, 8192, 12, 4, 0), False),
+    ((16, 5120, 8192, 12, 4, 0), True),
+    ((64, 5120, 448, 160, 8, 0), False),
+    ((128, 5120, 448, 160, 8, 0), True),
+    ((28, 5120, 704, 100, 5, 1), False),
+    ((31, 7168, 2048, 256, 8, 1), False),
+    ((32, 7168, 2048, 256, 8, 1), True),
+    # always from 64 slots per expert on
+    ((64, 256, 32, 1, 1, 0), True),
+    ((256, 1024, 512, 8, 2, 0), True),
+], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_gemm_regime_lines(shape, gemm):
+    T, H, I, E, k, sh = shape
+    names = _lib.load().phantom_moe_expert_kernels(T, H, I, E, k, sh).decode()
+    assert ("gemm" in names) == gemm, names
+
+
 def test_repack_and_permute_validation():
     lib = _lib.load()
     assert lib.phantom_q4_0_repack(FAKE, 15, 64, FAKE, FAKE, None) == EINVAL

@@ -103,28 +103,38 @@ def test_one_block_uses_every_xcd(dev):
     assert ms[0] < 0.7 * ms[1], ms
 
 
-# Just on either side of the line between the decode kernels and the GEMMs
-# below 64 slots per expert, for a shape of the token-tile kernels (12 slots
-# per expert) and one whose rows of H are too long for them (1 slot per expert)
+# Both sides of the lines between the decode kernels and the GEMMs below 64
+# slots per expert: token-tile shapes at 12, 14 and 16 slots per expert and at
+# 512, 320 and 160 * 1024 positions x I (by the kernel that would run down),
+# shapes whose rows of H are too long for those kernels at 225 * 1024
 LINE = [
-    (95, 256, 2048, 16, 2, False),
-    (96, 256, 2048, 16, 2, False),
-    (97, 256, 2048, 16, 2, True),
-    (31, 5376, 512, 128, 4, False),
-    (32, 5376, 512, 128, 4, True),
+    ((96, 256, 2048, 16, 2, False), False),
+    ((111, 256, 2048, 16, 2, False), False),
+    ((96, 256, 2048, 16, 2, True), True),
+    ((146, 320, 224, 32, 4, True), False),
+    ((147, 320, 224, 32, 4, True), True),
+    ((191, 2048, 768, 64, 4, False), False),
+    ((192, 2048, 768, 64, 4, False), True),
+    ((255, 1024, 480, 64, 4, False), False),
+    ((310, 1024, 480, 64, 4, True), True),
+    ((79, 384, 2048, 8, 2, False), False),
+    ((80, 384, 2048, 8, 2, False), True),
+    ((32, 5376, 512, 128, 4, True), False),
+    ((112, 5376, 512, 128, 4, False), False),
+    ((113, 5376, 512, 128, 4, False), True),
 ]
 
 
-@pytest.mark.parametrize("shape", LINE, ids=lambda s: "-".join(str(int(v)) for v in s))
-def test_regime_line(dev, shape):
+@pytest.mark.parametrize("shape,gemm", LINE, ids=lambda v: "-".join(map(str, map(int, v))) if isinstance(v, tuple) else "")
+def test_regime_line(dev, shape, gemm):
     from phantom_moe import _lib
 
     T, H, I, E, k, shared = shape
     names = _lib.load().phantom_moe_expert_kernels(T, H, I, E, k, int(shared)).decode()
-    assert ("gemm" in names) == (T * k >= (12 * E if H < 4096 else E)), names
+    assert ("gemm" in names) == gemm, names
     cfg = synth.MoEConfig("line", H, I, E, k, T, shared=shared)
     # the decode kernels' offset form loses about five times as much
-    run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg), room=1 if "gemm" in names else 8)
+    run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg), room=1 if gemm else 8)
 
 
 @pytest.mark.parametrize("T", [64, 130])  # the one-pass and (E 16) the two-pass router's copy of x
