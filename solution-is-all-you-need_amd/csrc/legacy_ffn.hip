@@ -395,33 +395,35 @@ __global__ __launch_bounds__(kLgWaves* kWave) void lg_down_kernel(const uint16_t
   }
 }
 
-// Active neuron list of one batch row per workgroup, in increasing order:
-// 16 neurons per thread, one 16-byte load where the row allows it, so a row of
-// 14336 takes one pass of the loop (four loads of single bytes and four passes
-// took 7.0 us, this 5.4).
+// Active neuron list of one batch row per workgroup, in increasing order: PER
+// neurons per thread, one load of PER bytes where the row allows it, and one
+// pass of the loop for most rows: 4 up to 4096 neurons, 16 beyond.  A row of
+// 14336 takes 5.4 us (7.0 in four passes of four byte loads); with 16 a row of
+// up to 4096 left most threads idle behind the others' 16 stores (the whole
+// predictor call at D 1024, two batch rows: 10.5 us with 4, 11.9 with 16).
+template <int PER>
 __global__ __launch_bounds__(kLgCompactThreads) void lg_compact_kernel(const uint8_t* __restrict__ mask,
                                                                        int32_t* __restrict__ idx,
                                                                        int32_t* __restrict__ count,
                                                                        int64_t D_ffn) {
   constexpr int kWaves = kLgCompactThreads / kWave;
-  constexpr int kPer = 16;
   __shared__ int s_wave[kWaves];
   const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
   const uint8_t* m = mask + (int64_t)blockIdx.x * D_ffn;
   int32_t* out = idx + (int64_t)blockIdx.x * D_ffn;
-  const bool vec = (reinterpret_cast<uintptr_t>(m) & 15u) == 0;
+  const bool vec = reinterpret_cast<uintptr_t>(m) % PER == 0;
   int64_t base = 0;
-  for (int64_t t0 = 0; t0 < D_ffn; t0 += kPer * kLgCompactThreads) {
-    const int64_t e0 = t0 + kPer * tid;
+  for (int64_t t0 = 0; t0 < D_ffn; t0 += PER * kLgCompactThreads) {
+    const int64_t e0 = t0 + PER * tid;
     uint32_t bits = 0;  // bit j: neuron e0 + j is active
-    if (vec && e0 + kPer <= D_ffn) {
-      const uint4 v = *reinterpret_cast<const uint4*>(m + e0);
-      const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+    if (vec && e0 + PER <= D_ffn) {
+      typedef uint32_t Words __attribute__((ext_vector_type(PER / 4)));
+      const Words q = *reinterpret_cast<const Words*>(m + e0);
 #pragma unroll
-      for (int j = 0; j < kPer; ++j) bits |= ((q[j / 4] >> (8 * (j % 4))) & 0xffu) != 0 ? 1u << j : 0u;
+      for (int j = 0; j < PER; ++j) bits |= (((uint32_t)q[j / 4] >> (8 * (j % 4))) & 0xffu) != 0 ? 1u << j : 0u;
     } else {
 #pragma unroll
-      for (int j = 0; j < kPer; ++j) {
+      for (int j = 0; j < PER; ++j) {
         const int64_t e = e0 + j;
         const uint8_t v = m[e < D_ffn ? e : D_ffn - 1];
         bits |= e < D_ffn && v != 0 ? 1u << j : 0u;
@@ -444,7 +446,7 @@ __global__ __launch_bounds__(kLgCompactThreads) void lg_compact_kernel(const uin
     }
     int64_t pos = base + before + incl - cnt;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j)
+    for (int j = 0; j < PER; ++j)
       if ((bits >> j) & 1u) out[pos++] = (int32_t)(e0 + j);
     base += total;
     __syncthreads();
@@ -651,8 +653,12 @@ PHANTOM_LEGACY_API float predict_active_neurons(const phantom_half* d_input, con
   p.mask = d_active_mask;
   hipError_t e = launch_lg_predict(p, stream);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(lg_compact_kernel, dim3(B), dim3(kLgCompactThreads), 0, stream, d_active_mask,
-                       d_active_indices, d_active_count, (int64_t)D_ffn);
+    if (D_ffn <= 4 * kLgCompactThreads)
+      hipLaunchKernelGGL(lg_compact_kernel<4>, dim3(B), dim3(kLgCompactThreads), 0, stream, d_active_mask,
+                         d_active_indices, d_active_count, (int64_t)D_ffn);
+    else
+      hipLaunchKernelGGL(lg_compact_kernel<16>, dim3(B), dim3(kLgCompactThreads), 0, stream, d_active_mask,
+                         d_active_indices, d_active_count, (int64_t)D_ffn);
     e = hipGetLastError();
   }
   if (e != hipSuccess) return (float)set_error(PHANTOM_MOE_ELAUNCH, "predict_active_neurons: %s", hipGetErrorString(e));

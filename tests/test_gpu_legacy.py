@@ -274,11 +274,12 @@ def test_calibrate_errors(dev):
         legacy.calibrate_sparsity_gate(x.half(), torch.zeros((4, 8), dtype=torch.float32, device=dev))
 
 
-@pytest.mark.parametrize("D_ffn", [1, 15, 16, 17, 1024, 16384, 16385, 20000])
+@pytest.mark.parametrize("D_ffn", [1, 15, 16, 17, 1024, 16384, 16385, 20000,
+                                   3, 4, 5, 4095, 4096, 4097, 4111, 4112, 4113])
 def test_compaction_edges(dev, D_ffn):
-    """Row lengths around the 16 neurons a thread takes and the 16384 of a pass,
-    in rows that start on and off a 16-byte boundary: indices increasing and
-    complete."""
+    """Row lengths around the neurons a thread takes (4 up to 4096, 16 beyond)
+    and the 16384 of a pass, in rows that start on and off the load's boundary:
+    indices increasing and complete."""
     B, D = 3, 8
     g = torch.Generator(device=dev).manual_seed(D_ffn)
     x = torch.randn(B, D, generator=g, device=dev).half()
