@@ -253,8 +253,8 @@ SMALL_CASES = [
     synth.MoEConfig("sigmoid_shared", 512, 128, 32, 4, 12, score="sigmoid", shared=True),
     synth.MoEConfig("zipf", 1024, 256, 128, 8, 32, zipf=1.1),
     synth.MoEConfig("k1", 128, 32, 4, 1, 3),
-    # 8800 slots: the many-workgroup permute, feeding the token-tile table and
-    # the shared expert (decode regime: 17 positions per expert on average)
+    # 8800 slots: the many-workgroup permute, feeding the GEMMs and the shared
+    # expert (17 positions per expert on average)
     synth.MoEConfig("many_slots_tiles", 256, 256, 512, 8, 1100, shared=True),
     # 16800 slots over 512 experts: 17 count blocks x 512 experts exceed the
     # fused scan's table, so the scan runs as its own launch
@@ -283,6 +283,30 @@ def test_moe_forward_small_vs_oracle(dev, cfg):
     np.testing.assert_array_equal(idx.cpu().numpy(), ridx)
     np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=1e-6, atol=1e-7)
     check_y(y.cpu().numpy(), ry, cfg.name)
+
+
+# Calls that stay on the decode kernels although they are large (short I, so
+# little work a position, or under 12 slots per expert): the many-workgroup
+# permute with the token-tile table, in the fused scan (9 count blocks x 512
+# experts) and as its own launch (17 blocks), for both kernels' tiles and for
+# down's alone (rows of H too long for the gate/up tile, whose K-split kernel
+# then reads more positions' tokens than its LDS holds); two-pass routing's bf16
+# copy of x (128 tokens or more)
+LARGE_DECODE = [
+    (synth.MoEConfig("tiles_fused_scan", 256, 32, 512, 8, 1100, shared=True), "gate_up_tile_kernel", "down_tile_kernel"),
+    (synth.MoEConfig("down_tiles_fused_scan", 4864, 32, 512, 8, 1100), "gate_up_kernel", "down_tile_kernel"),
+    (synth.MoEConfig("down_tiles_unfused_scan", 4864, 32, 512, 8, 2100, shared=True), "gate_up_kernel", "down_tile_kernel"),
+    (synth.MoEConfig("two_pass_tiles", 416, 288, 128, 8, 131), "gate_up_tile_kernel", "down_tile_kernel"),
+    (synth.MoEConfig("two_pass_tiles_shared", 512, 256, 128, 8, 190, score="sigmoid", shared=True),
+     "gate_up_tile_kernel", "down_tile_kernel"),
+]
+
+
+@pytest.mark.parametrize("cfg,gate_up,down", LARGE_DECODE, ids=lambda v: getattr(v, "name", ""))
+def test_large_decode_calls(dev, cfg, gate_up, down):
+    names = _lib.load().phantom_moe_expert_kernels(cfg.T, cfg.H, cfg.I, cfg.E, cfg.k, int(cfg.shared)).decode()
+    assert names == f"gate_up={gate_up};down={down}"
+    test_moe_forward_small_vs_oracle(dev, cfg)
 
 
 FULL = ["qwen3_decode_t1", "qwen3_decode_t32_zipf", "mixtral_decode_t1", "mixtral_decode_t16",
