@@ -46,7 +46,7 @@ CASES = [
     (129, 256, 64, 1, 1, False),    # a last block of one position
     (209, 384, 192, 2, 1, False),   # segments of any length
     (160, 640, 320, 2, 2, True),    # both experts and the shared one see every token
-    (1100, 512, 1024, 16, 1, False),  # a launch with drawn items
+    (1100, 512, 1024, 16, 1, False),  # segments of one or two blocks in down, items dealt
 ]
 
 
@@ -55,6 +55,26 @@ def test_gemm_edges(dev, shape):
     T, H, I, E, k, shared = shape
     cfg = synth.MoEConfig("gemm", H, I, E, k, T, shared=shared)
     run(dev, cfg, synth.activations(T, H, seed=T), synth.host_layer(cfg))
+
+
+# Launches of four rounds of items or more, whose items are drawn from the
+# ranges' counters: gate/up (a ragged last row block of I; H under 1024, where
+# the counters lie closer than a 128-byte line) and down (a ragged last row
+# block of H, K of three groups), on segments of uneven length
+@pytest.mark.parametrize("shape,rows,BM,per_cu", [((1100, 160, 8224, 16, 1, False), "I", 128, 2),
+                                                  ((1100, 416, 8224, 7, 1, True), "I", 128, 2),
+                                                  ((1100, 16416, 96, 16, 1, False), "H", 64, 3)],
+                         ids=["gate_up", "gate_up_shared", "down"])
+def test_drawn_items(dev, shape, rows, BM, per_cu):
+    T, H, I, E, k, shared = shape
+    cfg = synth.MoEConfig("drawn", H, I, E, k, T, shared=shared)
+    L, xb = synth.host_layer(cfg), synth.activations(T, H, seed=T)
+    idx = oracle.route(xb, L.router_w, k, cfg.score_mode)[0]
+    blocks = sum(-(-int(n) // BM) for n in np.bincount(idx.reshape(-1), minlength=E)) + (-(-T // BM) if shared else 0)
+    items = blocks * -(-(I if rows == "I" else H) // (64 if rows == "I" else 128))
+    # the grid is at most what is resident (expert_gemm.hip: kG2PerCu, kDrawRounds)
+    assert items >= 4 * per_cu * torch.cuda.get_device_properties(0).multi_processor_count, items
+    run(dev, cfg, xb, L)
 
 
 # Launches with few position blocks, whose item ranges are cut between row
