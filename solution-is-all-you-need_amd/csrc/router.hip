@@ -438,8 +438,12 @@ __device__ void prep_x_tile(const RouteK& a, int64_t t0, int TT, int part, int n
 
 // The GEMM regime's copy of one token: fp16 of x times the power of
 // two that puts the token's largest element in [2^14, 2^15), so every bf16
-// value down to 2^-32 of it is exact; the inverse goes to xs[t].  (Unscaled,
-// fp16 overflows from 65520 on and loses bits below 2^-17.)  A token with an
+// value down to 2^-31 of it is exact; the inverse goes to xs[t].  (Unscaled,
+// fp16 overflows from 65520 on and loses bits below 2^-17.)  The token is read
+// twice, for the largest element and for the copy, which costs the route some
+// microseconds over the decode kernels' one-pass copy (us: 8 experts at 48
+// tokens of H 4096 20.1 -> 27.0, 8 at 240 of H 3072 21.0 -> 24.8, 160 at 64 of
+// H 5120 29.7 -> 33.6, 141 at 918 of H 3200 68.4 -> 70.3).  A token with an
 // infinity or NaN is not scaled.  Layout [t][q][gi / 2][p][gi % 2][8]: the two
 // groups of half a quad are 128 consecutive bytes.
 // NT threads (tid of them; whole waves) share the token; with more than one
