@@ -1,6 +1,6 @@
 // expert_gemm.hip -- grouped int4 (Q4_0) expert SwiGLU FFN for gfx950 on the
-// matrix cores: every expert segment of a few positions or more runs as a GEMM
-// (gemm_regime).
+// matrix cores: calls of about a dozen positions per expert or more, with enough
+// work for the chip, run as GEMMs (gemm_regime).
 //
 // Reference operator: kernels/sparse_moe/sparse_matmul.cu:120-215 and its
 // dense branch (:322-365, cuBLAS GEMMs for gate/up and down, SwiGLU between),
