@@ -812,9 +812,7 @@ __global__ __launch_bounds__(256) void route_logits_big_kernel(RouteK a) {
   const int64_t t0 = (int64_t)blockIdx.y * TT;
   const int e0 = blockIdx.x * (4 * EW) + w * EW;
   const XT* x = static_cast<const XT*>(a.x);
-  if (a.prep_x && !a.prep_fp16)
-    prep_x_tile(a, t0, TT, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, (int)blockDim.x);
-  if (a.prep_x && a.prep_fp16)
+  if (a.prep_x)  // fewer than 16 experts and over 1024 tokens: always the GEMMs' copy
     for (int ti = (int)blockIdx.x * 4 + w; ti < TT && t0 + ti < a.T; ti += (int)gridDim.x * 4)
       prep_x_f16_token<kWave>(a, t0 + ti, lane, nullptr);
   if (a.counter && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.counter = 0;
